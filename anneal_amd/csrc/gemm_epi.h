@@ -95,7 +95,8 @@ __device__ __forceinline__ void epilogue_impl(const GemmDesc &d, const floatx16 
             }
         if (d.colsum) {
             cs += __shfl_xor(cs, 32, 64);
-            if (lane < 32 && nv) {
+            // a wave tile wholly past row M has no partial row: ceil(M / 32) rows is all the array holds
+            if (lane < 32 && nv && (FULL || mb < d.M)) {
                 if (d.colsum_ld) d.colsum[(long)(mb / 32) * d.colsum_ld + n] = cs;
                 else atomicAdd(d.colsum + n, cs);
             }
@@ -103,7 +104,8 @@ __device__ __forceinline__ void epilogue_impl(const GemmDesc &d, const floatx16 
     }
     if constexpr (EPI == EPI_MSE) {
         lossp = wave_sum(lossp);
-        if (lane == 0) {
+        // (likewise a loss partial past row M or column N: its cell would be another tile's, or past the array)
+        if (lane == 0 && (FULL || (mb < d.M && nb < d.N))) {
             if (d.loss_ld) d.lossacc[(long)(mb / 32) * d.loss_ld + nb / 32] = lossp;
             else atomicAdd(d.lossacc, lossp);
         }

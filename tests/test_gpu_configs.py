@@ -270,6 +270,30 @@ def test_config3_f16_mlp_step_vs_oracle(dev, shape):
         assert check_update(out[k], p[k], new[k], 2e-2), k
 
 
+@pytest.mark.parametrize("B,D,H,C", [(75, 32, 808, 126), (33, 40, 136, 20), (161, 64, 72, 12)])
+def test_mlp_gemm_step_tile_past_the_batch(dev, B, D, H, C):
+    """Batches whose last output tile has waves wholly past the last row: those have no partial row of the hidden bias
+    gradient to write (an odd number of 32-row blocks, with 64- and 128-row tiles)."""
+    p = data.mlp_ce_inputs(B, D, H, C, seed=21)
+    check_mlp(run_mlp_ce(dev, p, B, 0.01), p, 0.01)
+
+
+def test_config3_ragged_batch_and_output(dev):
+    """The same for the f16 step's bias-gradient rows and loss partials: 136 rows, 320 outputs."""
+    B, D0, D1, D2, D3 = 136, 128, 256, 192, 320
+    p = data.mlp3_inputs(B, D0, D1, D2, D3)
+    q = dict(p)
+    q["x"], q["t"] = data.f16_quantize(p["x"]), data.f16_quantize(p["t"])
+    _, g, _ = O.mlp3_step(q, 1e-3)
+    out = run_mlp3(dev, p, 1e-3)
+    h = np.maximum(q["x"] @ data.f16_quantize(p["W1"]).T, 0)
+    h = np.maximum(h @ data.f16_quantize(p["W2"]).T, 0)
+    want = np.sum((h @ data.f16_quantize(p["W3"]).T - q["t"]).astype(np.float64) ** 2)
+    assert abs(out["loss_sum"] - want) < 2e-2 * want
+    for k in ("dW1", "db1", "dW2", "db2", "dW3", "db3"):
+        assert O.relerr(out[k], g[k].ravel()) < 2e-2, k
+
+
 def test_config3_steps_bit_repeatable(dev):
     """The config-3 step has no float atomics (bias gradients and the loss are per-wave partials summed
     in a fixed order by the step tail), so re-running the same steps from the same state reproduces
