@@ -76,38 +76,99 @@ __global__ __launch_bounds__(256) void reduce_rows_kernel(const T *G, int M, int
     if (lane == 0) out[row] = op == RED_MAX ? acc : acc * scale;
 }
 
-// Column reduce, pass 1: block (column group of 64, row chunk) folds kRedRows rows with 4 row lanes per
-// column, then the 4 lanes in a fixed order; the chunk's value goes to part[chunk][n]. With Z, an element
-// enters as Where(Z == max(Z, 0), G, 0) (the ReLU backward mask, gradient_ruleset.go:153-161), else 0.
-template <typename T, typename TZ>
-__global__ __launch_bounds__(256) void reduce_cols_partial_kernel(const T *G, const TZ *Z, int M, int N, int op, float *part) {
-    __shared__ float red[4][64];
-    const int col = blockIdx.x * 64 + (threadIdx.x & 63), sub = threadIdx.x >> 6;
-    const int r0 = blockIdx.y * kRedRows, r1 = min(M, r0 + kRedRows);
-    float acc = red_init(op);
-    if (col < N)
-        for (int r = r0 + sub; r < r1; r += 4) {
-            const long i = (long)r * N + col;
-            float v = (float)G[i];
-            if (Z) v = (float)Z[i] >= 0.0f ? v : 0.0f;
-            acc = red_step(op, acc, v);
+// Column reduce. A row group of kColLanes lanes reads V consecutive columns per lane (16 bytes of G), so a block covers
+// kColLanes * V columns and 1024 / kColLanes = 64 rows at a time, four of each thread's rows in flight; the row groups are
+// then folded through LDS in row order (a fixed tree, so the result does not depend on timing). Bound by the read of G:
+// one column per lane and one row in flight took 7.8 us for 4096 x 1024 f16 (8 MiB), and the second pass, one thread per
+// column walking its chunks, 16.7 us; now 4.9 and 4.6 us (cold operands). With Z, an element enters as Where(Z == max(Z, 0), G, 0) (the
+// ReLU backward mask, gradient_ruleset.go:153-161), else 0.
+// Blocks take `rows` rows each. One chunk (gridDim.y = 1) writes out itself; more leave part[chunk][n] for the fold.
+constexpr int kColLanes = 16, kColThreads = 1024, kColGroups = kColThreads / kColLanes;
+template <typename T, int V>
+struct ColVec { typedef T type __attribute__((ext_vector_type(V))); };
+
+template <typename T, typename TZ, int V>
+__global__ __launch_bounds__(kColThreads) void reduce_cols_kernel(const T *G, const TZ *Z, int M, int N, int rows, int op,
+                                                                   float scale, float *part, float *out) {
+    typedef typename ColVec<T, V>::type vt;
+    typedef typename ColVec<TZ, V>::type vz;
+    __shared__ float red[kColGroups][kColLanes * V + 1];
+    const int l = threadIdx.x % kColLanes, grp = threadIdx.x / kColLanes;
+    const int c0 = blockIdx.x * (kColLanes * V) + l * V;
+    const int r0 = blockIdx.y * rows, r1 = min(M, r0 + rows);
+    float acc[V];
+#pragma unroll
+    for (int u = 0; u < V; u++) acc[u] = red_init(op);
+    if (c0 < N) {   // N % V == 0 (or V == 1): a lane's columns are all in or all out
+        for (int r = r0 + grp; r < r1; r += 4 * kColGroups) {
+            vt g[4];
+            vz z[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const long i = (long)min(r + j * kColGroups, r1 - 1) * N + c0;
+                g[j] = *(const vt *)(G + i);
+                if (Z) z[j] = *(const vz *)(Z + i);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if (r + j * kColGroups >= r1) break;
+#pragma unroll
+                for (int u = 0; u < V; u++) {
+                    float v = (float)g[j][u];
+                    if (Z) v = (float)z[j][u] >= 0.0f ? v : 0.0f;
+                    acc[u] = red_step(op, acc[u], v);
+                }
+            }
         }
-    red[sub][threadIdx.x & 63] = acc;
+    }
+#pragma unroll
+    for (int u = 0; u < V; u++) red[grp][l * V + u] = acc[u];
     __syncthreads();
-    if (sub == 0 && col < N) {
-        const int t = threadIdx.x;
-        part[(long)blockIdx.y * N + col] = red_join(op, red_join(op, red[0][t], red[1][t]), red_join(op, red[2][t], red[3][t]));
+    // fold: thread (column, eighth of the row groups), then the eighths in order
+    constexpr int CB = kColLanes * V, PARTS = 8;
+    __shared__ float red2[PARTS][CB];
+    for (int t = threadIdx.x; t < CB * PARTS; t += kColThreads) {
+        const int c = t % CB, p = t / CB;
+        float v = red[p * (kColGroups / PARTS)][c];
+#pragma unroll
+        for (int k = 1; k < kColGroups / PARTS; k++) v = red_join(op, v, red[p * (kColGroups / PARTS) + k][c]);
+        red2[p][c] = v;
+    }
+    __syncthreads();
+    const int col = blockIdx.x * CB + threadIdx.x;
+    if ((int)threadIdx.x < CB && col < N) {
+        float v = red2[0][threadIdx.x];
+#pragma unroll
+        for (int p = 1; p < PARTS; p++) v = red_join(op, v, red2[p][threadIdx.x]);
+        if (gridDim.y > 1) part[(long)blockIdx.y * N + col] = v;
+        else out[col] = op == RED_MAX ? v : v * scale;
     }
 }
 
-// Pass 2: out[n] = scale * fold of the chunk values in chunk order.
+// The chunks' fold: out[n] = scale * the chunk values of column n. A block takes 32 columns; its 8 row groups walk the
+// chunks 8 apart, 4 in flight, and are folded in order.
 __global__ __launch_bounds__(256) void reduce_cols_final_kernel(const float *part, int chunks, int N, int op,
                                                                  float scale, float *out) {
-    const int col = blockIdx.x * 256 + threadIdx.x;
-    if (col >= N) return;
-    float acc = chunks > 0 ? part[col] : red_init(op);   // an empty reduce yields the identity
-    for (int c = 1; c < chunks; c++) acc = red_join(op, acc, part[(long)c * N + col]);
-    out[col] = op == RED_MAX ? acc : acc * scale;
+    __shared__ float red[8][32];
+    const int l = threadIdx.x % 32, grp = threadIdx.x / 32, col = blockIdx.x * 32 + l;
+    float acc = red_init(op);   // an empty reduce yields the identity
+    if (col < N)
+        for (int c = grp; c < chunks; c += 32) {
+            float v[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = part[(long)min(c + 8 * j, chunks - 1) * N + col];
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (c + 8 * j < chunks) acc = red_join(op, acc, v[j]);
+        }
+    red[grp][l] = acc;
+    __syncthreads();
+    if (grp == 0 && col < N) {
+        float v = red[0][l];
+#pragma unroll
+        for (int k = 1; k < 8; k++) v = red_join(op, v, red[k][l]);
+        out[col] = op == RED_MAX ? v : v * scale;
+    }
 }
 
 // ── MaxPool2D ──────────────────────────────────────────────────────────────────────────────────────
@@ -293,23 +354,47 @@ hipError_t reduce_rows(const void *G, bool f16, int M, int N, int op, float scal
     return hipGetLastError();
 }
 
+template <typename T, typename TZ, int V>
+static hipError_t launch_reduce_cols(const void *G, const void *Z, int M, int N, int op, float scale, float *work,
+                                     float *out, hipStream_t s) {
+    // Chunks of 256 rows (4 per thread), doubled in number while the blocks stay within two per CU and a chunk keeps the
+    // kRedRows rows the workspace is sized for: few columns leave the chip to the rows. Up to 512 rows of few enough
+    // blocks go as one chunk: the second launch costs more than the longer walk (256 x 512 f32: 6.0 us as two launches
+    // of 64-row chunks, 4.2 us as one).
+    const int groups = (N + kColLanes * V - 1) / (kColLanes * V);
+    int rows = 4 * kColGroups;
+    if (M <= 512) rows = M;
+    else while (rows > kRedRows && (long)groups * ((M + rows - 1) / rows) < 512) rows /= 2;
+    const int chunks = (M + rows - 1) / rows;
+    hipLaunchKernelGGL((reduce_cols_kernel<T, TZ, V>), dim3(groups, chunks), dim3(kColThreads), 0, s, (const T *)G,
+                       (const TZ *)Z, M, N, rows, op, scale, work, out);
+    if (chunks > 1)
+        hipLaunchKernelGGL(reduce_cols_final_kernel, dim3((N + 31) / 32), dim3(256), 0, s, work, chunks, N, op, scale, out);
+    return hipGetLastError();
+}
+
+template <typename T, typename TZ>
+static hipError_t launch_reduce_cols_v(const void *G, const void *Z, int M, int N, int op, float scale, float *work,
+                                       float *out, hipStream_t s) {
+    // 16-byte loads of G (and 16- or 32-byte ones of Z) need every row to start on that boundary
+    constexpr int V = 16 / sizeof(T);
+    if (N % V == 0 && ((uintptr_t)G & 15) == 0 && ((uintptr_t)Z & (V * sizeof(TZ) >= 16 ? 15 : V * sizeof(TZ) - 1)) == 0)
+        return launch_reduce_cols<T, TZ, V>(G, Z, M, N, op, scale, work, out, s);
+    return launch_reduce_cols<T, TZ, 1>(G, Z, M, N, op, scale, work, out, s);
+}
+
 hipError_t reduce_cols(const void *G, bool f16, int M, int N, int op, float scale, float *work, float *out, hipStream_t s,
                        const void *Z, bool z_f16) {
     if (N <= 0) return hipSuccess;
-    const int chunks = M > 0 ? (M + kRedRows - 1) / kRedRows : 0;
-    const dim3 grid((N + 63) / 64, chunks), block(256);
-    if (chunks > 0) {
-        if (f16 && z_f16)
-            hipLaunchKernelGGL((reduce_cols_partial_kernel<half_t, half_t>), grid, block, 0, s, (const half_t *)G, (const half_t *)Z, M, N, op, work);
-        else if (f16)
-            hipLaunchKernelGGL((reduce_cols_partial_kernel<half_t, float>), grid, block, 0, s, (const half_t *)G, (const float *)Z, M, N, op, work);
-        else if (z_f16)
-            hipLaunchKernelGGL((reduce_cols_partial_kernel<float, half_t>), grid, block, 0, s, (const float *)G, (const half_t *)Z, M, N, op, work);
-        else
-            hipLaunchKernelGGL((reduce_cols_partial_kernel<float, float>), grid, block, 0, s, (const float *)G, (const float *)Z, M, N, op, work);
+    if (M <= 0) {
+        hipLaunchKernelGGL(reduce_cols_final_kernel, dim3((N + 31) / 32), dim3(256), 0, s, work, 0, N, op, scale, out);
+        return hipGetLastError();
     }
-    hipLaunchKernelGGL(reduce_cols_final_kernel, dim3((N + 255) / 256), dim3(256), 0, s, work, chunks, N, op, scale, out);
-    return hipGetLastError();
+    if (f16 && z_f16) return launch_reduce_cols_v<half_t, half_t>(G, Z, M, N, op, scale, work, out, s);
+    if (f16) return Z ? launch_reduce_cols_v<half_t, float>(G, Z, M, N, op, scale, work, out, s)
+                      : launch_reduce_cols_v<half_t, half_t>(G, Z, M, N, op, scale, work, out, s);
+    if (z_f16) return launch_reduce_cols_v<float, half_t>(G, Z, M, N, op, scale, work, out, s);
+    return launch_reduce_cols_v<float, float>(G, Z, M, N, op, scale, work, out, s);
 }
 
 hipError_t maxpool_fwd(const float *X, long NC, int H, int W, int kH, int kW, int sH, int sW, float *out, hipStream_t s) {

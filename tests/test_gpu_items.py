@@ -336,3 +336,28 @@ def test_reduce_template_rejects_bad_mask_keys(dev):
                 "tmpl:reduce;op=sum;axis=0;M=4;N=4;wza=1"):                # widening without the mask
         with pytest.raises(L.AnnealHipError):
             ex.run([ExecItem(key, bufs)], {1: np.ones(16, np.float32), 2: np.ones(16, np.float32)})
+
+
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("M,N", [(1, 1), (64, 10), (65, 128), (511, 136), (512, 130), (513, 136), (1000, 264), (4097, 8), (2100, 1)])
+def test_column_reduce_edges(dev, M, N, f16):
+    """Column reductions around the one-chunk limit (512 rows) and the edges of a 64- or 128-column block, with rows
+    that 16-byte loads divide and rows they do not: sums and sums of squares against float64 (an f32 sum of M terms in
+    a tree of depth about log2 M + 8 is within 24 * 2^-24 of its terms' absolute sum), maxima exactly, the ReLU mask."""
+    rng = np.random.default_rng(M * 1000 + N)
+    G, Z = (rng.standard_normal((M, N)).astype(np.float16 if f16 else np.float32).astype(np.float32) for _ in range(2))
+    dt, key = (L.AH_F16, "f16") if f16 else (L.AH_F32, "f32")
+    ex, g64 = Executor(dev), G.astype(np.float64)
+    for op in ("sum", "max", "sumsq"):
+        it = ExecItem(f"tmpl:reduce;dtype={key};op={op};axis=0;M={M};N={N};scale=0.5",
+                      [Buffer(10, N, [N]), Buffer(1, M * N, [M, N], dt)])
+        got = ex.run([it], {1: G.ravel()})[10]
+        if op == "max":
+            np.testing.assert_array_equal(got, G.max(0))
+        else:
+            t = g64 if op == "sum" else g64 * g64
+            assert np.all(np.abs(got - 0.5 * t.sum(0)) <= 24 * 2.0**-24 * 0.5 * np.abs(t).sum(0)), op
+    it = ExecItem(f"tmpl:reduce;dtype={key};op=sum;axis=0;M={M};N={N};pa=mask;in_a=1;za=2" + (";wza=1" if f16 else ""),
+                  [Buffer(10, N, [N]), Buffer(1, M * N, [M, N], dt), Buffer(2, M * N, [M, N], dt)])
+    got, t = ex.run([it], {1: G.ravel(), 2: Z.ravel()})[10], np.where(Z >= 0, g64, 0.0)
+    assert np.all(np.abs(got - t.sum(0)) <= 24 * 2.0**-24 * np.abs(t).sum(0))
