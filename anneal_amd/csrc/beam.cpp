@@ -87,7 +87,14 @@ int f16_variant_of(const G16Params &p) {
     return 0;
 }
 
-// Parses a gemm key and its current parameters (variant 0: the variant the shape selects by default).
+// The kernel a key without tuning parameters stands for in the seam: the compiler-scheduled class on the shape's tile
+// (256x256 when such tiles fill the chip, else 128x128), which every Opt edits from. (An unedited key runs
+// gemm16_default_variant's measured choice.)
+int seam_variant(const GemmDesc &d) {
+    return (long)((d.M + 255) / 256) * ((d.N + 255) / 256) >= 224 ? 3 : 1;
+}
+
+// Parses a gemm key and its current parameters (variant 0: seam_variant).
 int key_info(const std::string &key, KeyInfo *ki) {
     if (key.compare(0, 5, "tmpl:") != 0) return set_error(AH_ERR_UNSUPPORTED, "opts: not a template key");
     ki->kv = template_key_params(key, &ki->name);
@@ -101,7 +108,7 @@ int key_info(const std::string &key, KeyInfo *ki) {
             memset(&d, 0, sizeof d);
             auto dim = [&](const char *k) { auto it = ki->kv.find(k); return it == ki->kv.end() || it->second == "sym" ? 4096 : atoi(it->second.c_str()); };
             d.M = dim("M"); d.N = dim("N");
-            v = gemm16_default_variant(d);
+            v = seam_variant(d);
         }
         if (!gemm16_variant_params(v, &ki->knobs.p)) return set_error(AH_ERR_INVALID, "opts: variant %d", v);
         G16Params &p = ki->knobs.p;

@@ -64,13 +64,22 @@ bool gemm16_variant_params(int v, G16Params *out) {
     }
 }
 
+// The variant of a shape nothing has been tuned for. Measured with the layer epilogues (bias + ReLU, mask, SGD with the
+// gradient stored) on random operands that rotate through memory:
+//  - 256x256 tiles that fill the chip: 39 (16x16x32 MFMAs, DMAs between the MFMAs) against 3, the choice before:
+//    4096 x 4096 x 4096 107 / 116 / 150 us (NT / N,MN / MN,MN) against 123 / 158 / 190, x 1024 36.5 / 37.9 / 78 against
+//    43.5 / 42.3 / 86.
+//  - 128x128 tiles, at most one per CU: 35 (two k-groups, so two waves per SIMD) against 1: 4096 x 1024 x 4096
+//    39.3 / 40.1 / 44.2 us against 45.8 / 63.4 / 67.5, 2048 x 2048 x 2048 23.1 / 25.0 / 30.4 against 25.6 / 36.4 / 42.0.
+//    K must split into two groups of whole stages; otherwise 14 (four stages in flight): 40.9 / 41.8 / 47.0.
+//  - more 128x128 tiles than CUs: 1, whose 64 KiB of LDS let two tiles share a CU (35 and 14 hold 128 KiB): 2048 x 4096
+//    x 1024 24.0 / 27.8 / 39.8 us against 27.5 / 30.0 / 41.9.
 int gemm16_default_variant(const GemmDesc &d) {
-    int tile = d.tile;
-    if (tile == 0) {
-        long t256 = (long)((d.M + 255) / 256) * ((d.N + 255) / 256);
-        tile = t256 >= 224 ? 256 : 128;
-    }
-    return tile == 256 ? 3 : 1;
+    const long t256 = (long)((d.M + 255) / 256) * ((d.N + 255) / 256);
+    const long t128 = (long)((d.M + 127) / 128) * ((d.N + 127) / 128);
+    if (d.tile == 256 || (d.tile == 0 && t256 >= 224)) return 39;
+    if (t128 > 256) return 1;
+    return d.K % 128 == 0 ? 35 : 14;
 }
 
 // Returns true (and launches) when the shape/alignment admits the direct-to-LDS f16 kernel.
