@@ -735,9 +735,17 @@ struct Mlp3Trainer : ah_trainer {
                     if (rc == AH_OK) rc = ah_trainer_probe_read(this, &ms, &n);
                     if (rc == AH_OK && n > 0) t[v] = std::min(t[v], ms / n);
                 }
-            int bv = 1;
-            for (int v = 2; v <= kGemm16Variants; v++)
+            int bv = 1, one = 1;   // the fastest, and the fastest of one k-group
+            for (int v = 2; v <= kGemm16Variants; v++) {
                 if (t[v] < t[bv]) bv = v;
+                G16Params p;
+                if (gemm16_variant_params(v, &p) && p.kg == 1 && t[v] < t[one]) one = v;
+            }
+            // On an output of few tiles (up to 32 of 128x128: a few microseconds) one and two k-groups time alike, and
+            // which one wins is noise; they round differently, so one k-group is kept unless two are clearly faster: the
+            // step's bits then do not depend on the timing.
+            const GemmDesc g = gemm(i, false);
+            if ((long)((g.M + 127) / 128) * ((g.N + 127) / 128) <= 32 && t[one] <= 1.08 * t[bv]) bv = one;
             dev->gemm_variant[keys[i]] = bv;
         }
         probe_index = saved;
