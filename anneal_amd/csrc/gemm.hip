@@ -15,6 +15,7 @@
 // reduces (codegen/lower.go:667-716); products of f16 inputs are exact in f32.
 #include "ah_common.h"
 #include "gemm.h"
+#include "gemm16s.h"
 #include "gemm_epi.h"
 
 namespace ah {
@@ -511,6 +512,7 @@ hipError_t gemm_launch(const GemmDesc &d, hipStream_t s) {
     if (d.K < 0) return hipErrorInvalidValue;
     if (d.dtype == GEMM_F16) {
         hipError_t e = hipSuccess;
+        if (gemm16s_try_launch(d, s, &e)) return e;
         if (gemm16_try_launch(d, s, &e)) return e;
         if (d.A2) return hipErrorInvalidValue;   // two-plane contractions run on the direct-to-LDS kernels only
         return launch_layout<half_t>(d, s);

@@ -495,3 +495,80 @@ def test_gemm_f32_split_k_ragged(dev, cfg):
     got = Executor(dev).run([ExecItem(key, bufs)], {1: store_operand(A, 1).ravel(), 2: B.ravel(), 3: bias})[10]
     ref = np.maximum(A.astype(np.float64) @ B.astype(np.float64).T + bias, 0)
     assert O.relerr(got.reshape(M, N), ref) < 1e-5
+
+
+# Sizes around the split f16 kernel's edges: a tile and one more row, column or stage; K that ends inside a stage, inside a
+# 32-wide k-step, at one row (the weight gradient of one sample); outputs of one tile with K split many ways; 256-wide tiles.
+SPLIT_SHAPES = [(0, 0, 1, 64, 64), (0, 0, 3, 70, 2048), (0, 0, 32, 1000, 4104), (0, 0, 65, 129, 520), (0, 0, 200, 257, 72),
+                (0, 0, 999, 1000, 2056), (0, 0, 2100, 2056, 1000), (0, 1, 1, 64, 64), (0, 1, 33, 72, 2000), (0, 1, 130, 264, 136),
+                (0, 1, 1100, 520, 1000), (0, 1, 2100, 3080, 264), (1, 1, 64, 64, 1), (1, 1, 72, 136, 33), (1, 1, 264, 136, 4100),
+                (1, 1, 1000, 520, 77), (1, 1, 2056, 3080, 130)]
+
+
+@pytest.mark.parametrize("shape", SPLIT_SHAPES, ids=lambda s: "ta%d_tb%d_%dx%dx%d" % s)
+def test_gemm16_split_kernel_edges(dev, shape):
+    """Every epilogue of the untuned f16 contraction against float64 at sizes that are no multiple of a tile. The f32 sums
+    of K products are within (K + 16) * 2^-24 of the sum of their magnitudes; f16 results add a rounding each (2^-11 of the
+    value, twice with a bias). Memory past the output stays as it was, and a repeat gives the same bits (the partials of a
+    split K are added in split order)."""
+    ta, tb, M, N, K = shape
+    rng = np.random.default_rng(M + N + K)
+    A, B = (q16(rng.standard_normal(s)) for s in ((M, K), (N, K)))
+    bias, aux, W = q16(rng.standard_normal(N)), q16(rng.standard_normal((M, N))), rng.standard_normal((M, N)).astype(np.float32)
+    aux = np.where(aux < 0, np.float32(-0.0), aux)
+    ref, mag = A.astype(np.float64) @ B.astype(np.float64).T, np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64).T
+    acc = (K + 16) * 2.0**-24 * mag
+    half = lambda v: v.astype(np.float16)   # noqa: E731
+    As, Bs = store_operand(A, ta), store_operand(B, tb)
+    pad = 64
+    bufs = dict(A=dev.buffer(half(As), L.AH_F16), B=dev.buffer(half(Bs), L.AH_F16))
+    dC = dev.buffer(np.full(M * N + pad, 7, np.float16), L.AH_F16)
+    dbias, daux = dev.buffer(half(bias), L.AH_F16), dev.buffer(half(aux), L.AH_F16)
+    kw = dict(dtype=L.AH_F16, ta=ta, tb=tb, M=M, N=N, K=K, lda=As.shape[1], ldb=Bs.shape[1], ldc=N, **bufs)
+
+    def f16_out(**e):
+        dev.gemm(C_out=dC, **kw, **e)
+        one = dC.read()
+        dev.gemm(C_out=dC, **kw, **e)
+        two = dC.read()
+        np.testing.assert_array_equal(one.view(np.uint16), two.view(np.uint16))
+        assert np.all(one[M * N:] == 7)
+        return one[:M * N].astype(np.float64).reshape(M, N)
+
+    tiny = 2.0**-24   # half the smallest f16 step
+    C = f16_out(epi=L.EPI_STORE, scale=0.5)
+    assert np.all(np.abs(C - 0.5 * ref) <= 0.5 * acc + 2.0**-11 * np.abs(C) + 2 * tiny)
+    z = ref + bias
+    C = f16_out(epi=L.EPI_BIAS_RELU, bias=dbias)
+    slack = acc + 2.0**-11 * (np.abs(ref) + np.abs(z)) * 1.01 + 4 * tiny
+    assert np.all(np.abs(C - np.maximum(z, 0)) <= slack)
+    sure = np.abs(z) > slack
+    assert np.array_equal((np.signbit(C) & (C == 0))[sure], (z < 0)[sure])
+    dead = np.signbit(aux) & (aux == 0)
+    C = f16_out(epi=L.EPI_MASK, aux=daux, ldaux=N, scale=1.0)
+    assert np.all(np.abs(C - np.where(dead, 0.0, ref)) <= acc + 2.0**-11 * np.abs(C) + 2 * tiny)
+    dW, dg, dW16 = dev.buffer(W), dev.buffer(np.full(M * N + pad, 7, np.float32)), dev.buffer(M * N, L.AH_F16)
+    dev.gemm(epi=L.EPI_SGD, scale=0.25, lr=0.5, W32=dW, W16=dW16, gout=dg, **kw)
+    g, Wn = dg.read(), dW.read().reshape(M, N)
+    assert np.all(g[M * N:] == 7)
+    g = g[:M * N].reshape(M, N)
+    assert np.all(np.abs(g - 0.25 * ref) <= 0.25 * acc + 2.0**-24 * np.abs(g))
+    assert np.all(np.abs(Wn - (W - 0.5 * g.astype(np.float64))) <= 2.0**-23 * (np.abs(Wn) + np.abs(g)))
+    np.testing.assert_array_equal(dW16.read(), Wn.astype(np.float16).ravel())
+    for b in (*bufs.values(), dC, dbias, daux, dW, dg, dW16):
+        b.free()
+
+
+def test_gemm16_split_kernel_unaligned_output(dev):
+    """A row stride that 16-byte accesses do not divide (ldc 77) and an operand with a padded stride."""
+    M, N, K, ldc, lda = 70, 75, 200, 77, 208
+    rng = np.random.default_rng(3)
+    A, B = q16(rng.standard_normal((M, lda))), q16(rng.standard_normal((N, K)))
+    dA, dB = dev.buffer(A.astype(np.float16), L.AH_F16), dev.buffer(B.astype(np.float16), L.AH_F16)
+    dC = dev.buffer(np.full(M * ldc, 7, np.float16), L.AH_F16)
+    dev.gemm(dtype=L.AH_F16, epi=L.EPI_STORE, ta=0, tb=0, M=M, N=N, K=K, A=dA, B=dB, lda=lda, ldb=K, C_out=dC, ldc=ldc)
+    C = dC.read().astype(np.float64).reshape(M, ldc)
+    ref = A[:, :K].astype(np.float64) @ B.astype(np.float64).T
+    assert np.all(np.abs(C[:, :N] - ref) <= 2.0**-11 * np.abs(ref) + 1e-3) and np.all(C[:, N:] == 7)
+    for b in (dA, dB, dC):
+        b.free()
