@@ -1306,7 +1306,8 @@ int ah_chain_step(ah_device *dev, const float *X, const float *g, int32_t R, int
         return set_error(AH_ERR_INVALID, "ah_chain_step: bad argument (Cc must be a multiple of 4)");
     float *w = nullptr;
     AH_HIP(hipMalloc(&w, (size_t)chain_workspace_floats(R, Cc) * 4));
-    hipError_t e = hipMemsetAsync(w, 0, 256, dev->stream);   // the resident path's arrival counter
+    hipError_t e = hipMemsetAsync(w, 0, 256, dev->stream);   // the strip kernel's counters
+    if (e == hipSuccess) e = hipMemsetAsync(w + chain_array_floats(R, Cc), 0, (size_t)chain_sync_ints(Cc) * 4, dev->stream);
     if (e == hipSuccess) e = chain_step(X, g, R, Cc, w, dX, dg, loss, dev->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(dev->stream);
     hipFree(w);
@@ -1318,12 +1319,12 @@ int ah_chain_step_noalloc(ah_device *dev, const float *X, const float *g, int32_
                           float *loss) {
     if (!dev || !X || !g || !dX || !dg || !loss || R <= 0 || Cc <= 0 || Cc % 4)
         return set_error(AH_ERR_INVALID, "ah_chain_step_noalloc: bad argument (Cc must be a multiple of 4)");
-    const long need = chain_workspace_floats(R, Cc), cap = chain_scratch_floats();
+    const long need = chain_array_floats(R, Cc), cap = chain_scratch_floats();
     if (need > cap)
         return set_error(AH_ERR_INVALID, "ah_chain_step_noalloc: R=%d x Cc=%d needs %ld workspace floats, the maximum is %ld",
                          R, Cc, need, cap);
     if (!dev->chain_scratch) return set_error(AH_ERR_INVALID, "ah_chain_step_noalloc: device has no chain workspace");
-    AH_HIP(chain_step(X, g, R, Cc, dev->chain_scratch, dX, dg, loss, dev->stream));
+    AH_HIP(chain_step(X, g, R, Cc, dev->chain_scratch, dX, dg, loss, dev->stream, -1, (int *)(dev->chain_scratch + cap)));
     return AH_OK;
 }
 

@@ -358,108 +358,69 @@ __global__ __launch_bounds__(256) void chain_grad_kernel(const float *X, int R, 
     }
 }
 
-// ── config 5 in one pass over HBM: strips of X held on chip ─────────────────────
-// Every softmax / RMS row of the chain is one column of X, and dg, the loss terms and dX of a column
-// need only that column. So one workgroup per CU takes a strip of 16 columns x R rows (R = 4096 or
-// 8192: up to 512 KiB), keeps all of it on chip (kResRegs float4 per thread in VGPRs, kResLds in LDS through
-// LDS-DMA), and runs the whole chain on it: the column max, sum e, sum e^2 and the tie count
-// (accumulated while the strip lands, see below), the per-column scalars of chain_finalize, dg, and dX
-// written once from the on-chip copy. HBM sees X read once and dX written once; the three-kernel chain reads X
-// twice and moves its column partials through memory. Thread t owns columns c0 + 4 (t & 3) .. + 3 of
-// rows (t >> 2) + 128 i. Every sum is a fixed tree (slots in order, then lanes by xor, then waves in
-// order), so results are deterministic. Each workgroup stores its 16 columns' loss terms summed in
-// column order; the last to arrive (arrival counter, zero before and after the launch) adds the strips'
-// sums in strip order.
-constexpr int kResThreads = 512, kResRowLanes = kResThreads / 4, kResCols = 16;
-constexpr int kResMaxRegs = 45, kResMaxLds = 19;   // float4 slots per thread in VGPRs / in LDS (152 KiB)
+// ── the chain in one pass over HBM: strips of X held on chip ──────────────────────
+// Every softmax / RMS row of the chain is one column of X, and dg, the loss terms and dX of a column need only that column.
+// A strip of 32 columns (128 bytes of a row: one cache line) is held on chip by `parts` workgroups of consecutive row
+// ranges, up to 4096 rows (512 KiB) each: NS float4 slots per thread, 45 in VGPRs and the rest in LDS through LDS-DMA. Each
+// workgroup takes its rows' column statistics (max, sum e, sum e^2, ties) while they land; with several parts they are
+// exchanged once through memory, 512 bytes a part; then every workgroup evaluates the column's scalars and writes its rows
+// of dX from the on-chip copy. HBM sees X read once and dX written once, where the three-kernel chain reads X twice.
+//
+// Bound by HBM, load phase then store phase. Strips of 16 columns, one workgroup of 8192 rows each, took 70.5 us for 8192 x
+// 4096 with X in memory (49 us with X left in the Infinity Cache by the step before): 64-byte row segments use half of each
+// line, and only a neighbour on the same XCD can use the rest.
+//
+// Waiting for the other parts is bounded: a workgroup that has polled `spin` times takes the missing statistics from X
+// itself, in the same order, so the result is the same and nothing depends on the parts running together.
+//
+// Thread t owns columns 4 (t & 7) .. + 3 of rows (t >> 3) + 64 i of its range: slot 0 the last, possibly partial 64 rows,
+// slots 1 .. nfull the whole ones. Every sum is a fixed tree (slots in order, then lanes by xor, waves in order, parts in
+// order). Part 0 stores the strip's loss sum; the last strip to arrive (counter, zero before and after) adds them in order.
+constexpr int kStripThreads = 512, kStripWaves = kStripThreads / 64, kStripCols = 32, kStripRows = kStripThreads / 8;
+constexpr int kStripMaxRegs = 45, kStripMaxSlots = 64;   // float4 slots per thread in VGPRs; in all (19 in LDS: 152 KiB)
+constexpr int kStripMaxParts = 16, kStripMaxPartsFull = 4;   // parts whose statistics fit beside the held rows in LDS
+constexpr int kStripMaxStrips = 1024;                    // arrival counters of ah_chain_step_noalloc's workspace
+constexpr int kStripSpin = 1 << 14;
 
-__device__ __forceinline__ float res_tree_max(float v) {   // over the 16 lanes of a wave with equal lane & 3
-    v = fmaxf(v, __shfl_xor(v, 4, 64));
+__device__ __forceinline__ float strip_tree_max(float v) {   // over the 8 lanes of a wave with equal lane & 7
     v = fmaxf(v, __shfl_xor(v, 8, 64));
     v = fmaxf(v, __shfl_xor(v, 16, 64));
     return fmaxf(v, __shfl_xor(v, 32, 64));
 }
-__device__ __forceinline__ float res_tree_sum(float v) {
-    v += __shfl_xor(v, 4, 64);
+__device__ __forceinline__ float strip_tree_sum(float v) {
     v += __shfl_xor(v, 8, 64);
     v += __shfl_xor(v, 16, 64);
     return v + __shfl_xor(v, 32, 64);
 }
 
-// NS: float4 slots per thread, R = 128 * NS rows.
-template <int NS>
-__global__ __launch_bounds__(kResThreads) void chain_resident_kernel(const float *X, int R, int Cc, const float *g,
-                                                                      float *dX, float *dg, float *lossp, int *counter,
-                                                                      float *loss) {
-    constexpr int kResRegs = NS < kResMaxRegs ? NS : kResMaxRegs, kResLds = NS - kResRegs;
-    static_assert(kResLds <= kResMaxLds, "the strip does not fit on chip");
-    __shared__ __attribute__((aligned(1024))) floatx4 held[kResLds > 0 ? kResLds : 1][kResThreads];
-    __shared__ float red[4][kResThreads / 64][kResCols];               // per wave: max, sum e, sum e^2, ties
-    __shared__ __attribute__((aligned(16))) float coef[6][kResCols];   // dX factors A, B, column max, -, tie share, loss term
-    __shared__ int ticket;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int nstrips = Cc / kResCols;
-    int strip = blockIdx.x;
-    if ((nstrips & 7) == 0) strip = (strip & 7) * (nstrips >> 3) + (strip >> 3);   // neighbouring strips share an XCD
-    const int q = tid & 3, rl = tid >> 2;
-    // Buffer accesses from the strip's first column: the lane's offset in one VGPR, the slot's row
-    // offset (wave-uniform) in the scalar offset, so the 64 slots cost no address registers. The
-    // caller guarantees R * Cc * 4 < 2^31.
-    typedef unsigned u4 __attribute__((ext_vector_type(4)));
-    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void *)(X + strip * kResCols), (short)0, 0x7fffffff, 0x00020000);
-    const __amdgpu_buffer_rsrc_t dr = __builtin_amdgcn_make_buffer_rsrc((void *)(dX + strip * kResCols), (short)0, 0x7fffffff, 0x00020000);
-    const int voff = (rl * Cc + 4 * q) * 4;
-    const int rstepB = kResRowLanes * Cc * 4;
-    // 1. the strip: register slots first (they are consumed first), then the LDS slots
-    floatx4 v[kResRegs];
+// A thread's running statistics of its four columns: the reference mt its exponentials are taken against, sum e, sum e^2,
+// the exact running max and the count of elements equal to it. An element more than 2^60 above mt (where e^2 could
+// overflow) first moves the reference to itself.
+struct StripStat {
+    float mt[4], se[4], sq[4], mr[4], cnt[4];
+    __device__ __forceinline__ void init(const float (&ref)[4]) {
 #pragma unroll
-    for (int i = 0; i < kResRegs; i++)
-        v[i] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(xr, voff, i * rstepB, 0));
-#pragma unroll
-    for (int j = 0; j < kResLds; j++)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void *)&held[j][wave * 64], 16,
-                                                     voff, (kResRegs + j) * rstepB, 0, 0);
-    // 2-3. Statistics while the strip lands. Each thread takes a provisional max mt of its own first
-    // kProv slots, then, slot by slot as the loads arrive, adds e = 2^(x/ln2 - mt/ln2) and e^2 to its
-    // column sums and keeps the exact running max with the count of elements equal to it. Once every
-    // slot has landed, the column max m is the max of the running maxima, the tie count the sum of the
-    // counts of the threads whose running max is m, and each thread's sums are rescaled by
-    // 2^((mt - m_w)/ln2) to its wave's max m_w, each wave's by 2^((m_w - m)/ln2) to the column max.
-    // x stays in place; the dX pass recomputes e against m. An element more than 2^60 above the
-    // thread's reference (where e^2 could overflow) first moves the reference to itself, rescaling the
-    // thread's sums (no such element occurs unless the strip's values grow by a factor e^41 along the
-    // column).
-    constexpr int kProv = 8;
-    static_assert(kResRegs >= kProv, "the provisional max takes register slots");
-    float mt[4] = {-FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX};
-#pragma unroll
-    for (int i = 0; i < kProv; i++)
-#pragma unroll
-        for (int u = 0; u < 4; u++) mt[u] = fmaxf(mt[u], v[i][u]);
-    float mct[4], mr[4], cnt[4], se[4] = {}, sq[4] = {};
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-        mct[u] = mt[u] * AH_INV_LN2;
-        mr[u] = -FLT_MAX;
-        cnt[u] = 0.0f;
+        for (int u = 0; u < 4; u++) {
+            mt[u] = ref[u];
+            se[u] = sq[u] = cnt[u] = 0.0f;
+            mr[u] = -FLT_MAX;
+        }
     }
-    auto stat = [&](const floatx4 &x) {
+    __device__ __forceinline__ void push(const floatx4 &x) {
         float d[4];
 #pragma unroll
-        for (int u = 0; u < 4; u++) d[u] = __builtin_fmaf(x[u], AH_INV_LN2, -mct[u]);
-        // one wave-uniform test per slot for the (never taken on ordinary data) re-base
+        for (int u = 0; u < 4; u++) d[u] = (x[u] - mt[u]) * AH_INV_LN2;
         const float dm = fmaxf(fmaxf(d[0], d[1]), fmaxf(d[2], d[3]));
-        if (__builtin_amdgcn_ballot_w64(dm > 60.0f)) {
+        if (__builtin_amdgcn_ballot_w64(dm > 60.0f)) {   // wave-uniform, never taken on ordinary data
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
+            for (int u = 0; u < 4; u++)
                 if (d[u] > 60.0f) {
                     const float f = fast_exp2(-d[u]);
                     se[u] *= f;
                     sq[u] *= f * f;
-                    mct[u] = x[u] * AH_INV_LN2;
-                    d[u] = __builtin_fmaf(x[u], AH_INV_LN2, -mct[u]);
+                    mt[u] = x[u];
+                    d[u] = 0.0f;
                 }
-            }
         }
 #pragma unroll
         for (int u = 0; u < 4; u++) {
@@ -467,59 +428,207 @@ __global__ __launch_bounds__(kResThreads) void chain_resident_kernel(const float
             se[u] += e;
             sq[u] += e * e;
             const float mn = fmaxf(mr[u], x[u]);
-            cnt[u] = (mn == mr[u] ? cnt[u] : 0.0f) + (x[u] == mn ? 1.0f : 0.0f);   // count of the running max
+            cnt[u] = (mn == mr[u] ? cnt[u] : 0.0f) + (x[u] == mn ? 1.0f : 0.0f);
             mr[u] = mn;
         }
-        // materialise the running values after every slot (left free, the compiler runs one sum over
-        // all slots before the next, keeping every slot's e live in between)
+        // materialise the running values after every slot (left free, the compiler runs one sum over all slots before the
+        // next, keeping every slot's e live in between)
         asm volatile("" : "+v"(se[0]), "+v"(se[1]), "+v"(se[2]), "+v"(se[3]), "+v"(sq[0]), "+v"(sq[1]), "+v"(sq[2]),
                      "+v"(sq[3]), "+v"(cnt[0]), "+v"(cnt[1]), "+v"(cnt[2]), "+v"(cnt[3]), "+v"(mr[0]), "+v"(mr[1]),
                      "+v"(mr[2]), "+v"(mr[3]));
-    };
-#pragma unroll
-    for (int i = 0; i < kResRegs; i++) stat(v[i]);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's LDS-DMA has landed (each lane reads its own)
-#pragma unroll 2
-    for (int j = 0; j < kResLds; j++) {
-        const floatx4 x = *(volatile floatx4 *)&held[j][tid];
-        stat(x);
     }
-    // 4. Column statistics in one cross-wave round: each wave folds its 16 lanes of a column (max,
-    // then the sums rescaled to the wave's max, the tie count at that max) and lanes 0-3 post the
-    // wave's (max, sum e, sum e^2, ties) per column; thread c < 16 folds the 8 waves of column c in
-    // order, rescaling each wave's sums to the column max, and evaluates the column's scalars
-    // (chain_finalize's rules); every thread then reads its 4 columns' scalars back.
-    float m[4];
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-        m[u] = res_tree_max(mr[u]);                    // the wave's max of the column
-        const float f = fast_exp2(mct[u] - m[u] * AH_INV_LN2);   // 2^((mt - m_w)/ln2) <= 1
-        se[u] = res_tree_sum(se[u] * f);
-        sq[u] = res_tree_sum(sq[u] * (f * f));
-        cnt[u] = res_tree_sum(mr[u] == m[u] ? cnt[u] : 0.0f);
-    }
-    if (lane < 4)
+    // the wave's statistics of its columns to red[..][wave][column]: max, then the sums rescaled to it, ties at it
+    __device__ __forceinline__ void post(float (*red)[kStripWaves][kStripCols], int wave, int lane) {
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-            red[0][wave][4 * lane + u] = m[u];
-            red[1][wave][4 * lane + u] = se[u];
-            red[2][wave][4 * lane + u] = sq[u];
-            red[3][wave][4 * lane + u] = cnt[u];
+            const float m = strip_tree_max(mr[u]);
+            const float f = fast_exp2((mt[u] - m) * AH_INV_LN2);
+            const float s = strip_tree_sum(se[u] * f), q = strip_tree_sum(sq[u] * (f * f));
+            const float t = strip_tree_sum(mr[u] == m ? cnt[u] : 0.0f);
+            if (lane < 8) {
+                red[0][wave][4 * lane + u] = m;
+                red[1][wave][4 * lane + u] = s;
+                red[2][wave][4 * lane + u] = q;
+                red[3][wave][4 * lane + u] = t;
+            }
         }
+    }
+};
+
+// n statistics of a column (max, sum e, sum e^2, ties, the sums against their own max) folded in order; at(k, i) reads them.
+template <class At>
+__device__ __forceinline__ void strip_fold(int n, At &&at, float (&o)[4]) {
+    float m = at(0, 0);
+    for (int i = 1; i < n; i++) m = fmaxf(m, at(0, i));
+    float s = 0.0f, q = 0.0f, t = 0.0f;
+    for (int i = 0; i < n; i++) {
+        const float mi = at(0, i);
+        const float f = fast_exp2((mi - m) * AH_INV_LN2);
+        s += at(1, i) * f;
+        q += at(2, i) * (f * f);
+        t += mi == m ? at(3, i) : 0.0f;
+    }
+    o[0] = m; o[1] = s; o[2] = q; o[3] = t;
+}
+
+// part_rows: rows per part (a multiple of 64, at most 64 * NS; the last part may have fewer). stats: parts * 128 floats a
+// strip. sync: two counters a strip, arrivals and departures, zero before and after.
+template <int NS>
+__global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float *X, int R, int Cc, int parts, int part_rows,
+                                                                     const float *g, float *dX, float *dg, float *stats,
+                                                                     int *sync, float *lossp, int *counter, float *loss,
+                                                                     int spin) {
+    constexpr int kRegs = NS < kStripMaxRegs ? NS : kStripMaxRegs, kLds = NS - kRegs, kProv = NS < 8 ? NS : 8;
+    constexpr int kParts = NS > kStripMaxRegs ? kStripMaxPartsFull : kStripMaxParts;
+    __shared__ __attribute__((aligned(1024))) floatx4 held[kLds > 0 ? kLds : 1][kStripThreads];
+    __shared__ float red[4][kStripWaves][kStripCols];
+    __shared__ float pstat[4][kParts][kStripCols];
+    __shared__ __attribute__((aligned(16))) float coef[5][kStripCols];   // dX factors A, B, column max, tie share, loss term
+    __shared__ int flag;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int nstrips = (Cc + kStripCols - 1) / kStripCols;
+    // runs of (strip, part) per XCD: a strip's parts start together, and neighbouring strips, which share lines where Cc is
+    // no multiple of 32, meet in one L2
+    const int L = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    if (L >= nstrips * parts) return;
+    const int strip = L / parts, part = L - strip * parts;
+    const int q = tid & 7, rl = tid >> 3, c0 = strip * kStripCols, col = c0 + 4 * q;
+    const bool colok = col < Cc;   // Cc % 4 == 0: all four columns or none
+    const int rbeg = part * part_rows, rows = min(part_rows, R - rbeg), nfull = (rows - 1) / kStripRows;
+    const int row0 = nfull * kStripRows + rl;   // slot 0's row
+    const bool ok0 = row0 < rows && colok;
+    // Buffer accesses from the part's first row and the strip's first column: the lane's offset in one VGPR, the slot's row
+    // offset (wave-uniform) in the scalar offset. Lanes without a row or column and slots past nfull get an offset past the
+    // descriptor's size: loads give zeros, stores do nothing. The caller guarantees R * Cc * 4 < 2^31.
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    constexpr int kOut = (int)0x80000000;
+    const long org = (long)rbeg * Cc + c0;
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void *)(X + org), (short)0, 0x7fffffff, 0x00020000);
+    const __amdgpu_buffer_rsrc_t dr = __builtin_amdgcn_make_buffer_rsrc((void *)(dX + org), (short)0, 0x7fffffff, 0x00020000);
+    const int voff = colok ? (rl * Cc + 4 * q) * 4 : kOut, voff0 = ok0 ? (row0 * Cc + 4 * q) * 4 : kOut;
+    const int rstepB = kStripRows * Cc * 4;
+    // 1. the rows: register slots first (they are consumed first), then the LDS slots
+    floatx4 v[kRegs];
+    v[0] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(xr, voff0, 0, 0));
+    // the row offset is a running value advanced through an empty asm, here and for the stores, so that only the current one
+    // is live (all of them kept overflow the SGPRs into VGPR lanes)
+    int soff = 0;
+#pragma unroll
+    for (int i = 1; i < kRegs; i++) {
+        v[i] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(xr, i <= nfull ? voff : kOut, soff, 0));
+        soff += rstepB;
+        asm volatile("" : "+s"(soff));
+    }
+#pragma unroll
+    for (int j = 0; j < kLds; j++) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void *)&held[j][wave * 64], 16,
+                                                     kRegs + j <= nfull ? voff : kOut, soff, 0, 0);
+        soff += rstepB;
+        asm volatile("" : "+s"(soff));
+    }
+    // 2. statistics while they land, against the max of the thread's first slots
+    StripStat st;
+    {
+        float ref[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) ref[u] = ok0 ? v[0][u] : -FLT_MAX;
+#pragma unroll
+        for (int i = 1; i < kProv; i++)
+            if (i <= nfull)
+#pragma unroll
+                for (int u = 0; u < 4; u++) ref[u] = fmaxf(ref[u], v[i][u]);
+        st.init(ref);
+    }
+    if (ok0) st.push(v[0]);
+#pragma unroll
+    for (int i = 1; i < kRegs; i++)
+        if (i <= nfull) st.push(v[i]);
+    if constexpr (kLds > 0) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's LDS-DMA has landed (each lane reads its own)
+#pragma unroll 2
+        for (int j = 0; j < kLds; j++) {
+            if (kRegs + j > nfull) break;
+            const floatx4 x = *(volatile floatx4 *)&held[j][tid];
+            st.push(x);
+        }
+    }
+    st.post(red, wave, lane);
     __syncthreads();
-    if (tid < kResCols) {
-        float mm = red[0][0][tid];
-        for (int w = 1; w < kResThreads / 64; w++) mm = fmaxf(mm, red[0][w][tid]);
-        const float mmc = mm * AH_INV_LN2;
-        float s_ = 0.0f, q_ = 0.0f, t_ = 0.0f;
-        for (int w = 0; w < kResThreads / 64; w++) {
-            const float mw = red[0][w][tid];
-            const float f = fast_exp2(__builtin_fmaf(mw, AH_INV_LN2, -mmc));
-            s_ += red[1][w][tid] * f;
-            q_ += red[2][w][tid] * (f * f);
-            t_ += mw == mm ? red[3][w][tid] : 0.0f;
+    // 3. the part's column statistics, and the other parts'
+    float own[4];
+    if (tid < kStripCols) strip_fold(kStripWaves, [&](int k, int w) { return red[k][w][tid]; }, own);
+    if (parts > 1) {
+        float *const mine = stats + ((long)strip * parts + part) * (4 * kStripCols);
+        int *const arrive = sync + 2 * strip;
+        if (wave == 0) {
+            if (lane < kStripCols)
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    __hip_atomic_store(mine + k * kStripCols + lane, own[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // performed where the XCDs are coherent, before the arrival
+            if (lane == 0) {
+                __hip_atomic_fetch_add(arrive, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                int got = __hip_atomic_load(arrive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                for (int k = 0; k < spin && got < parts; k++) {
+                    __builtin_amdgcn_s_sleep(4);
+                    got = __hip_atomic_load(arrive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+                flag = got >= parts;
+            }
         }
-        const int c = strip * kResCols + tid;
+        __syncthreads();
+        if (flag) {
+            if (tid < kStripCols)
+                for (int p = 0; p < parts; p++)
+#pragma unroll
+                    for (int k = 0; k < 4; k++)
+                        pstat[k][p][tid] = __hip_atomic_load(stats + ((long)strip * parts + p) * (4 * kStripCols) + k * kStripCols + tid,
+                                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } else {
+            // the same statistics from memory, slot for slot in the order their own workgroup takes them
+            for (int p = 0; p < parts; p++) {
+                const int pb = p * part_rows, pr = min(part_rows, R - pb), pf = (pr - 1) / kStripRows, r0 = pf * kStripRows + rl;
+                const bool pok = r0 < pr && colok;
+                const float *const px = X + (long)pb * Cc + col;
+                auto at = [&](int i) { return colok ? *(const floatx4 *)(px + (long)((i - 1) * kStripRows + rl) * Cc) : (floatx4){}; };
+                const floatx4 x0 = pok ? *(const floatx4 *)(px + (long)r0 * Cc) : (floatx4){};
+                float ref[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) ref[u] = pok ? x0[u] : -FLT_MAX;
+                for (int i = 1; i < kProv && i <= pf; i++) {
+                    const floatx4 x = at(i);
+#pragma unroll
+                    for (int u = 0; u < 4; u++) ref[u] = fmaxf(ref[u], x[u]);
+                }
+                StripStat o;
+                o.init(ref);
+                if (pok) o.push(x0);
+                for (int i = 1; i <= pf; i++) o.push(at(i));
+                __syncthreads();   // red is read by the fold before
+                o.post(red, wave, lane);
+                __syncthreads();
+                if (tid < kStripCols) {
+                    float f[4];
+                    strip_fold(kStripWaves, [&](int k, int w) { return red[k][w][tid]; }, f);
+#pragma unroll
+                    for (int k = 0; k < 4; k++) pstat[k][p][tid] = f[k];
+                }
+            }
+        }
+        if (tid < kStripCols) strip_fold(parts, [&](int k, int p) { return pstat[k][p][tid]; }, own);
+        if (tid == 0) {   // the last part to leave (every one has arrived by then) clears the counters for the next launch
+            const int gone = __hip_atomic_fetch_add(arrive + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (gone == parts - 1) {
+                __hip_atomic_store(arrive, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(arrive + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+    }
+    // 4. the column's scalars (chain_finalize's rules), the same in every part
+    if (tid < kStripCols) {
+        const int c = c0 + tid;
+        const bool live = c < Cc;
+        const float mm = own[0], s_ = own[1], q_ = own[2], t_ = own[3];
         const float eps = 1e-6f, rR = 1.0f / (float)R;
         const float r_s = 1.0f / s_;
         const float sumS = s_ * r_s;
@@ -527,7 +636,7 @@ __global__ __launch_bounds__(kResThreads) void chain_resident_kernel(const float
         const float qm = sqq * rR;
         const float T = sqrtf(qm + eps);
         const float r = 1.0f / T;
-        const float gi = g[c];
+        const float gi = live ? g[c] : 0.0f;
         const float gR = gi * sumS;
         const float gT = ((-gR) * r) * r;
         const float gu = gT * (1.0f / (2.0f * T));
@@ -535,75 +644,63 @@ __global__ __launch_bounds__(kResThreads) void chain_resident_kernel(const float
         const float gRs = (gi * r) * s_ + 2.0f * gsq_ * (r_s * q_);
         const float gs_ = ((-gRs) * r_s) * r_s;
         const float gm = -(AH_LN2 * AH_INV_LN2) * (r_s * gRs + gs_ * s_);
-        // dX = e * (gr * r_s + gs) + e^2 * (2 gsq r_s^2), plus the tie share where x is the max: the
-        // per-element backward of S = e * r_s through sum e and sum S^2, with its per-column factors
-        // gathered (the reference's op order rounds them per element; the difference is at f32 rounding)
+        // dX = e * (gr * r_s + gs) + e^2 * (2 gsq r_s^2), plus the tie share where x is the max: the per-element backward
+        // of S = e * r_s through sum e and sum S^2, with its per-column factors gathered (the reference's op order rounds
+        // them per element; the difference is at f32 rounding)
         coef[0][tid] = (gi * r) * r_s + gs_;
         coef[1][tid] = 2.0f * gsq_ * (r_s * r_s);
-        coef[4][tid] = gm * (1.0f / t_);
-        coef[5][tid] = gi * (r * sumS);
         coef[2][tid] = mm;
-        dg[c] = r * sumS;
+        coef[3][tid] = gm * (1.0f / t_);
+        coef[4][tid] = live ? gi * (r * sumS) : 0.0f;
+        if (part == 0 && live) dg[c] = r * sumS;
     }
     __syncthreads();
-    float ca[4], cb[4], sh[4], mc[4];
+    // 5. dX from the held rows
     {
         const floatx4 a = *(const floatx4 *)&coef[0][4 * q], b = *(const floatx4 *)&coef[1][4 * q],
-                      mx = *(const floatx4 *)&coef[2][4 * q], e = *(const floatx4 *)&coef[4][4 * q];
+                      mx = *(const floatx4 *)&coef[2][4 * q], sh = *(const floatx4 *)&coef[3][4 * q];
+        auto put = [&](const floatx4 &x, int off, int soff) {
+            floatx4 o;
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            ca[u] = a[u];
-            cb[u] = b[u];
-            m[u] = mx[u];
-            mc[u] = mx[u] * AH_INV_LN2;
-            sh[u] = e[u];
+            for (int u = 0; u < 4; u++) {
+                const float e = fast_exp2((x[u] - mx[u]) * AH_INV_LN2);
+                o[u] = (a[u] + b[u] * e) * e + (x[u] == mx[u] ? sh[u] : 0.0f);
+            }
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, o), dr, off, soff, 0);
+            // Wait states after the 16-byte store before anything may rewrite its data registers: without them a VALU
+            // write two instructions later, behind a v_readlane of a spilled SGPR, reached memory in some lanes.
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("s_nop 4" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        put(v[0], voff0, 0);
+        soff = 0;
+#pragma unroll
+        for (int i = 1; i < kRegs; i++) {
+            if (i <= nfull) put(v[i], voff, soff);
+            soff += rstepB;
+            asm volatile("" : "+s"(soff));
+        }
+        // the LDS slots through volatile loads: else the compiler may keep an earlier pass's reads live for this one
+#pragma unroll 2
+        for (int j = 0; j < kLds; j++) {
+            if (kRegs + j > nfull) break;
+            const floatx4 x = *(volatile floatx4 *)&held[j][tid];
+            put(x, voff, soff);
+            soff += rstepB;
+            asm volatile("" : "+s"(soff));
         }
     }
-    // 5. dX from the held strip: the register slots, then the LDS slots two at a time. The LDS slots are
-    // read through volatile loads in every pass: otherwise the compiler may keep one pass's reads live in
-    // registers for the next, which the held strip leaves no room for.
-    auto each = [&](auto &&f) {
-#pragma unroll
-        for (int i = 0; i < kResRegs; i++) f(i, v[i]);
-#pragma unroll 2
-        for (int j = 0; j < kResLds; j++) {
-            const floatx4 x = *(volatile floatx4 *)&held[j][tid];
-            f(kResRegs + j, x);
-        }
-    };
-    // The stores' row offset is a running value advanced through an empty asm after each slot, so only
-    // the current one is live (all 64 kept from the loads overflow the SGPRs into VGPR lanes).
-    int soff = 0;
-    each([&](int i, const floatx4 &x) {
-        floatx4 o;
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const float e = fast_exp2(__builtin_fmaf(x[u], AH_INV_LN2, -mc[u]));
-            const float gzs = (ca[u] + cb[u] * e) * e;
-            o[u] = gzs + (x[u] == m[u] ? sh[u] : 0.0f);
-        }
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, o), dr, voff, soff, 0);
-        soff += rstepB;
-        asm volatile("" : "+s"(soff));
-        // Wait states after the 16-byte store before anything may rewrite its data registers. Without
-        // them the compiler placed a VALU write to the store's first data VGPR two instructions later,
-        // behind a v_readlane of a spilled SGPR, and that dword of some lanes was stored already
-        // overwritten (observed: element 0 of the float4 in lanes 12-15 of a wave).
-        __builtin_amdgcn_sched_barrier(0);
-        asm volatile("s_nop 4" ::: "memory");
-        __builtin_amdgcn_sched_barrier(0);
-    });
-    // 6. loss: this strip's 16 terms in column order, then the strips in order by the last to arrive
-    __syncthreads();
+    // 6. loss: the strip's 32 terms in column order, then the strips in order by the last to arrive
+    if (part != 0) return;
     if (tid == 0) {
         float a = 0.0f;
-        for (int c = 0; c < kResCols; c++) a += coef[5][c];
+        for (int c = 0; c < kStripCols; c++) a += coef[4][c];
         __hip_atomic_store(lossp + strip, a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        ticket = ticket_take_atomic_partials(counter);   // lossp[] is written and read as atomics
+        flag = ticket_take_atomic_partials(counter);   // lossp[] is written and read as atomics
     }
     __syncthreads();
-    if (ticket != (int)gridDim.x - 1 || wave != 0) return;
-    // lane k adds strips k*P .. k*P+P-1 in order, then the lanes in a fixed tree
+    if (flag != nstrips - 1 || wave != 0) return;
     const int per = (nstrips + 63) / 64;
     float a = 0.0f;
     for (int k = 0; k < per; k++) {
@@ -617,21 +714,50 @@ __global__ __launch_bounds__(kResThreads) void chain_resident_kernel(const float
     }
 }
 
-// Row counts with an instantiated strip program: R = 8192 (64 float4 slots per thread: 45 in VGPRs, 19 in
-// LDS) and R = 4096 (32, all in VGPRs); other shapes take the three-kernel chain.
-bool chain_resident_fits(int R, int Cc) {
-    return (R == 128 * 64 || R == 128 * 32) && Cc >= kResCols && Cc % kResCols == 0 && (long)R * Cc * 4 < (1L << 31);
+// Parts per strip and rows per part: as few parts as hold the rows on chip, then more while the workgroups stay within one
+// per CU and each keeps 8 slots (512 rows: less leaves a workgroup nothing to overlap its fixed cost with).
+struct StripPlan {
+    int parts, rows;
+};
+static StripPlan strip_plan(int R, int Cc) {
+    const int strips = (Cc + kStripCols - 1) / kStripCols;
+    auto slots = [&](int parts) { return ((R + parts - 1) / parts + kStripRows - 1) / kStripRows; };
+    int parts = 1;
+    while (parts < kStripMaxParts && slots(parts) > kStripMaxSlots) parts++;
+    while (parts < kStripMaxParts && strips * (parts + 1) <= 256 && slots(parts + 1) >= 8) parts++;
+    const int rows = slots(parts) * kStripRows;
+    return {(R + rows - 1) / rows, rows};
 }
 
-hipError_t chain_resident(const float *X, const float *g, int R, int Cc, float *lossp, int *counter, float *dX, float *dg,
-                          float *loss, hipStream_t s) {
+bool chain_resident_fits(int R, int Cc) {
+    if (R <= 0 || Cc <= 0 || Cc % 4 || (long)R * Cc * 4 >= (1L << 31)) return false;
+    if ((Cc + kStripCols - 1) / kStripCols > kStripMaxStrips) return false;
+    const StripPlan p = strip_plan(R, Cc);
+    return p.rows <= kStripRows * (p.parts <= kStripMaxPartsFull ? kStripMaxSlots : kStripMaxRegs);
+}
+
+template <int NS>
+static void launch_strip(const float *X, const float *g, int R, int Cc, const StripPlan &p, float *stats, int *sync, float *lossp,
+                         int *counter, float *dX, float *dg, float *loss, int spin, hipStream_t s) {
+    const int wgs = (Cc + kStripCols - 1) / kStripCols * p.parts;
+    hipLaunchKernelGGL(chain_strip_kernel<NS>, dim3((wgs + 7) / 8 * 8), dim3(kStripThreads), 0, s, X, R, Cc, p.parts, p.rows, g,
+                       dX, dg, stats, sync, lossp, counter, loss, spin);
+}
+
+hipError_t chain_resident(const float *X, const float *g, int R, int Cc, float *arrays, int *sync, int *counter, float *dX,
+                          float *dg, float *loss, int spin, hipStream_t s) {
     if (!chain_resident_fits(R, Cc)) return hipErrorInvalidValue;
-    if (R == 128 * 64)
-        hipLaunchKernelGGL(chain_resident_kernel<64>, dim3(Cc / kResCols), dim3(kResThreads), 0, s, X, R, Cc, g, dX, dg,
-                           lossp, counter, loss);
-    else
-        hipLaunchKernelGGL(chain_resident_kernel<32>, dim3(Cc / kResCols), dim3(kResThreads), 0, s, X, R, Cc, g, dX, dg,
-                           lossp, counter, loss);
+    const StripPlan p = strip_plan(R, Cc);
+    const int strips = (Cc + kStripCols - 1) / kStripCols, slots = p.rows / kStripRows;
+    float *lossp = arrays + (p.parts > 1 ? (long)strips * p.parts * 4 * kStripCols : 0);
+#define AH_STRIP(n) launch_strip<n>(X, g, R, Cc, p, arrays, sync, lossp, counter, dX, dg, loss, spin, s)
+    if (slots <= 4) AH_STRIP(4);
+    else if (slots <= 8) AH_STRIP(8);
+    else if (slots <= 16) AH_STRIP(16);
+    else if (slots <= 32) AH_STRIP(32);
+    else if (slots <= kStripMaxRegs) AH_STRIP(kStripMaxRegs);
+    else AH_STRIP(kStripMaxSlots);
+#undef AH_STRIP
     return hipGetLastError();
 }
 
@@ -825,20 +951,25 @@ hipError_t mse_finalize(const float *acc, float scale, float *out, hipStream_t s
     return hipGetLastError();
 }
 
-// Workspace: word 0 is the resident path's arrival counter (zero before the first call, left zero by
-// every call; the three-kernel path never touches it), then from float 64 either path's arrays.
+// Workspace: word 0 is the strip kernel's loss counter, zero before the first call and left zero by every call; from float
+// 64 either path's arrays; then the strips' arrival counters (likewise zero between calls; the three-kernel path touches
+// neither). ah_chain_step_noalloc, whose arrays serve every shape, keeps the arrival counters apart.
 constexpr long kChainHead = 64;
-long chain_workspace_floats(int R, int Cc) {
+long chain_array_floats(int R, int Cc) {
     int nch = (R + kChainStatsRows - 1) / kChainStatsRows;
     const long three = (long)nch * Cc * 4 + (long)Cc * 8 + (Cc + kFinCols - 1) / kFinCols;
-    return kChainHead + std::max(three, (long)(Cc / kResCols));
+    const long strips = (Cc + kStripCols - 1) / kStripCols;   // their loss terms, and the parts' statistics
+    return kChainHead + std::max(three, chain_resident_fits(R, Cc) ? strips * (1 + 4L * kStripCols * strip_plan(R, Cc).parts) : 0L);
 }
+long chain_sync_ints(int Cc) { return 2L * ((Cc + kStripCols - 1) / kStripCols); }
+long chain_workspace_floats(int R, int Cc) { return chain_array_floats(R, Cc) + chain_sync_ints(Cc); }
 
 hipError_t chain_step(const float *X, const float *g, int R, int Cc, float *work, float *dX, float *dg, float *loss,
-                      hipStream_t s, int phase) {
+                      hipStream_t s, int phase, int *sync, int spin) {
     if (Cc % 4 != 0 || R <= 0) return hipErrorInvalidValue;
     if (phase < 0 && chain_resident_fits(R, Cc))
-        return chain_resident(X, g, R, Cc, work + kChainHead, (int *)work, dX, dg, loss, s);
+        return chain_resident(X, g, R, Cc, work + kChainHead, sync ? sync : (int *)(work + chain_array_floats(R, Cc)), (int *)work, dX,
+                              dg, loss, spin < 0 ? kStripSpin : spin, s);
     work += kChainHead;
     const int nch = (R + kChainStatsRows - 1) / kChainStatsRows;
     const int nfin = (Cc + kFinCols - 1) / kFinCols;
@@ -873,7 +1004,7 @@ namespace ah {
 namespace {
 constexpr long kChainScratchFloats = 1L << 22;   // 16 MiB: R x Cc up to 16320 x 4096 (config 5, 8192 x 4096, needs 2.13M floats)
 constexpr int kMaxDevices = 64;
-static __device__ __align__(256) float scratch[kChainScratchFloats];
+static __device__ __align__(256) float scratch[kChainScratchFloats + 2 * kStripMaxStrips];   // arrays, then arrival counters
 float *g_scratch_ptr[kMaxDevices];
 }  // namespace
 

@@ -552,6 +552,7 @@ int template_chain(const Params &P, TemplateKernel *t) {
     GET("R", R, false);
     GET("Cc", Cc, false);
     if (R.v <= 0 || Cc.v <= 0 || Cc.v % 4) return set_error(AH_ERR_INVALID, "tmpl chain: Cc must be a positive multiple of 4");
+    const int spin = (int)P.integer("spin", -1);   // polls for the other parts of a strip (-1: the default)
     t->side = {{3, false}, {4, false}};
     t->bytes = [R, Cc](int64_t) -> std::vector<int64_t> {
         const int64_t x = R.v * Cc.v * 4;
@@ -563,7 +564,7 @@ int template_chain(const Params &P, TemplateKernel *t) {
         if (int rc = need(key.c_str(), n_ptrs, 5)) return rc;
         if (int rc = ensure_ws(self, chain_workspace_floats((int)R.v, (int)Cc.v) * 4)) return rc;
         AH_HIP(chain_step((const float *)ptrs[1], (const float *)ptrs[2], (int)R.v, (int)Cc.v, (float *)self->ws,
-                          (float *)ptrs[0], (float *)ptrs[3], (float *)ptrs[4], d->stream));
+                          (float *)ptrs[0], (float *)ptrs[3], (float *)ptrs[4], d->stream, -1, nullptr, spin));
         return AH_OK;
     };
     return AH_OK;

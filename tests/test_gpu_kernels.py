@@ -9,6 +9,7 @@ import pytest
 
 import oracle_lib as O
 from anneal_amd import _lib as L
+from anneal_amd.executor import Buffer, ExecItem, Executor
 
 pytestmark = pytest.mark.gpu
 RNG = np.random.default_rng(99)
@@ -165,6 +166,47 @@ def test_chain_kernel_vs_oracle(dev, R, Cc, grow):
     assert abs(dl.read()[0] - wl) < 1e-5 * abs(wl)
     for b in (dXb, dgb, dX, dg, dl):
         b.free()
+
+
+# Row counts around the strip kernel's slots (64 rows), parts (4096 rows, or fewer for few columns) and instances; columns
+# that end inside a 32-column strip, one strip, more strips than CUs; beyond its reach (40960 rows: the three-kernel chain)
+@pytest.mark.parametrize("R,Cc", [(1, 4), (64, 36), (65, 32), (513, 64), (1025, 100), (2049, 260), (2881, 8200), (3001, 2052),
+                                  (4097, 64), (5000, 132), (8192, 96), (9000, 8), (16384, 32), (40960, 4)])
+@pytest.mark.parametrize("spin", [-1, 0])
+def test_chain_strip_edges(dev, R, Cc, spin):
+    """The chain item against the float64 closed form and, bit for bit, against itself with spin = 0: there a workgroup
+    whose strip's other parts have not arrived takes their statistics from X itself. -FLT_MAX entries (a mask) and a
+    column of them, where every element ties, and a jump far above the first rows."""
+    rng = np.random.default_rng(R + Cc)
+    X = rng.standard_normal((R, Cc)).astype(np.float32)
+    X[:, 1] = np.float32(-3.4028234663852886e38) if R > 1 else X[:, 1]
+    X[: R // 3, 2] = np.float32(-3.4028234663852886e38)
+    X[R // 2:, 3] += 100.0
+    g = (1 + 0.02 * rng.standard_normal(Cc)).astype(np.float32)
+    ex = Executor(dev)
+
+    def run(spin):
+        bufs = [Buffer(10, R * Cc, [R, Cc]), Buffer(1, R * Cc, [R, Cc]), Buffer(2, Cc, [Cc]), Buffer(11, Cc, [Cc]), Buffer(12, 1, [1])]
+        key = f"tmpl:chain;R={R};Cc={Cc}" + (f";spin={spin}" if spin >= 0 else "")
+        return ex.run([ExecItem(key, bufs)], {1: X.ravel(), 2: g})
+
+    out = run(spin)
+    x = X.astype(np.float64)
+    m = x.max(0)
+    e = np.exp(x - m)
+    S = e / e.sum(0)
+    T = np.sqrt((S * S).mean(0) + 1e-6)
+    dg = 1 / T
+    gS = g / T - S * (g * S.sum(0) / (R * T**3))
+    dX = S * (gS - (gS * S).sum(0))
+    got = out[10].reshape(R, Cc)
+    # An f32 evaluation forms dX = S (gS - sum gS S) from terms of S g / T that nearly cancel, a few roundings each; at the
+    # maxima the tie share adds what is left of g / T - g / T: an ulp of it after each of four roundings.
+    assert np.all(np.abs(got - dX) <= 16 * 2.0**-23 * (S * g / T) + 4 * 2.0**-24 * (g / T) * (x == m) + 1e-30)
+    assert np.allclose(out[11], dg, rtol=1e-5) and np.allclose(out[12][0], (g * dg).sum(), rtol=1e-5)
+    if spin == 0:
+        for k, v in run(-1).items():
+            np.testing.assert_array_equal(out[k].view(np.uint32), v.view(np.uint32))
 
 
 F16_VARIANTS = list(range(1, 40))   # every gemm16 variant (gemm16_kernel.h Var<V>; 32-39 use 16x16x32 MFMAs)
