@@ -393,18 +393,22 @@ __device__ __forceinline__ float strip_tree_sum(float v) {
     return v + __shfl_xor(v, 32, 64);
 }
 
-// A thread's running statistics of its four columns: the reference mt its exponentials are taken against, sum e, sum e^2,
-// the exact running max and the count of elements equal to it. An element more than 2^60 above mt (where e^2 could
-// overflow) first moves the reference to itself.
+// A thread's running statistics of its four columns: the reference mt its exponentials are taken against, sum e, sum e^2
+// and the exact running max. An element more than 2^60 above mt (where e^2 could overflow) first moves the reference to
+// itself. The elements equal to the max are counted afterwards, and only where a lane met its running max again (a bit of
+// `tie`, kept in scalar registers): counting them as they land took 5 of 17 vector operations per element, in a kernel whose
+// vector work shows (8192 x 4096: 67.3 us with the count, 59.1 us without any statistics).
 struct StripStat {
-    float mt[4], se[4], sq[4], mr[4], cnt[4];
+    float mt[4], se[4], sq[4], mr[4];
+    uint64_t tie;
     __device__ __forceinline__ void init(const float (&ref)[4]) {
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             mt[u] = ref[u];
-            se[u] = sq[u] = cnt[u] = 0.0f;
+            se[u] = sq[u] = 0.0f;
             mr[u] = -FLT_MAX;
         }
+        tie = 0;
     }
     __device__ __forceinline__ void push(const floatx4 &x) {
         float d[4];
@@ -427,18 +431,30 @@ struct StripStat {
             const float e = fast_exp2(d[u]);
             se[u] += e;
             sq[u] += e * e;
-            const float mn = fmaxf(mr[u], x[u]);
-            cnt[u] = (mn == mr[u] ? cnt[u] : 0.0f) + (x[u] == mn ? 1.0f : 0.0f);
-            mr[u] = mn;
+            tie |= __builtin_amdgcn_ballot_w64(x[u] == mr[u]);
+            mr[u] = fmaxf(mr[u], x[u]);
         }
         // materialise the running values after every slot (left free, the compiler runs one sum over all slots before the
         // next, keeping every slot's e live in between)
         asm volatile("" : "+v"(se[0]), "+v"(se[1]), "+v"(se[2]), "+v"(se[3]), "+v"(sq[0]), "+v"(sq[1]), "+v"(sq[2]),
-                     "+v"(sq[3]), "+v"(cnt[0]), "+v"(cnt[1]), "+v"(cnt[2]), "+v"(cnt[3]), "+v"(mr[0]), "+v"(mr[1]),
-                     "+v"(mr[2]), "+v"(mr[3]));
+                     "+v"(sq[3]), "+v"(mr[0]), "+v"(mr[1]), "+v"(mr[2]), "+v"(mr[3]));
+    }
+    // the elements equal to the thread's max, counted over each(f) (f is called with every element of the thread) where any
+    // lane of the wave may have more than one; some: the thread has an element at all
+    template <class Each>
+    __device__ __forceinline__ void count(bool some, float (&cnt)[4], Each &&each) const {
+#pragma unroll
+        for (int u = 0; u < 4; u++) cnt[u] = some ? 1.0f : 0.0f;
+        if (tie == 0) return;
+#pragma unroll
+        for (int u = 0; u < 4; u++) cnt[u] = 0.0f;
+        each([&](const floatx4 &x) {
+#pragma unroll
+            for (int u = 0; u < 4; u++) cnt[u] += x[u] == mr[u] ? 1.0f : 0.0f;
+        });
     }
     // the wave's statistics of its columns to red[..][wave][column]: max, then the sums rescaled to it, ties at it
-    __device__ __forceinline__ void post(float (*red)[kStripWaves][kStripCols], int wave, int lane) {
+    __device__ __forceinline__ void post(float (*red)[kStripWaves][kStripCols], int wave, int lane, const float (&cnt)[4]) {
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             const float m = strip_tree_max(mr[u]);
@@ -469,6 +485,12 @@ __device__ __forceinline__ void strip_fold(int n, At &&at, float (&o)[4]) {
         t += mi == m ? at(3, i) : 0.0f;
     }
     o[0] = m; o[1] = s; o[2] = q; o[3] = t;
+}
+
+// i <= nfull, compared anew at each use: all 64 of a thread's comparisons kept for the later passes overflow the SGPRs.
+__device__ __forceinline__ bool strip_in(int i, int nfull) {
+    asm volatile("" : "+s"(nfull));
+    return i <= nfull;
 }
 
 // part_rows: rows per part (a multiple of 64, at most 64 * NS; the last part may have fewer). stats: parts * 128 floats a
@@ -515,14 +537,14 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
     int soff = 0;
 #pragma unroll
     for (int i = 1; i < kRegs; i++) {
-        v[i] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(xr, i <= nfull ? voff : kOut, soff, 0));
+        v[i] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(xr, strip_in(i, nfull) ? voff : kOut, soff, 0));
         soff += rstepB;
         asm volatile("" : "+s"(soff));
     }
 #pragma unroll
     for (int j = 0; j < kLds; j++) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void *)&held[j][wave * 64], 16,
-                                                     kRegs + j <= nfull ? voff : kOut, soff, 0, 0);
+                                                     strip_in(kRegs + j, nfull) ? voff : kOut, soff, 0, 0);
         soff += rstepB;
         asm volatile("" : "+s"(soff));
     }
@@ -534,7 +556,7 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
         for (int u = 0; u < 4; u++) ref[u] = ok0 ? v[0][u] : -FLT_MAX;
 #pragma unroll
         for (int i = 1; i < kProv; i++)
-            if (i <= nfull)
+            if (strip_in(i, nfull))
 #pragma unroll
                 for (int u = 0; u < 4; u++) ref[u] = fmaxf(ref[u], v[i][u]);
         st.init(ref);
@@ -542,7 +564,7 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
     if (ok0) st.push(v[0]);
 #pragma unroll
     for (int i = 1; i < kRegs; i++)
-        if (i <= nfull) st.push(v[i]);
+        if (strip_in(i, nfull)) st.push(v[i]);
     if constexpr (kLds > 0) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's LDS-DMA has landed (each lane reads its own)
 #pragma unroll 2
@@ -552,7 +574,18 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
             st.push(x);
         }
     }
-    st.post(red, wave, lane);
+    float cnt[4];
+    st.count(colok && (nfull > 0 || ok0), cnt, [&](auto &&f) {
+        if (ok0) f(v[0]);
+#pragma unroll
+        for (int i = 1; i < kRegs; i++)
+            if (strip_in(i, nfull)) f(v[i]);
+        for (int j = 0; j < kLds && kRegs + j <= nfull; j++) {
+            const floatx4 x = *(volatile floatx4 *)&held[j][tid];
+            f(x);
+        }
+    });
+    st.post(red, wave, lane, cnt);
     __syncthreads();
     // 3. the part's column statistics, and the other parts'
     float own[4];
@@ -604,8 +637,12 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
                 o.init(ref);
                 if (pok) o.push(x0);
                 for (int i = 1; i <= pf; i++) o.push(at(i));
+                o.count(colok && (pf > 0 || pok), cnt, [&](auto &&f) {
+                    if (pok) f(x0);
+                    for (int i = 1; i <= pf; i++) f(at(i));
+                });
                 __syncthreads();   // red is read by the fold before
-                o.post(red, wave, lane);
+                o.post(red, wave, lane, cnt);
                 __syncthreads();
                 if (tid < kStripCols) {
                     float f[4];
@@ -664,7 +701,13 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
 #pragma unroll
             for (int u = 0; u < 4; u++) {
                 const float e = fast_exp2((x[u] - mx[u]) * AH_INV_LN2);
-                o[u] = (a[u] + b[u] * e) * e + (x[u] == mx[u] ? sh[u] : 0.0f);
+                o[u] = (a[u] + b[u] * e) * e;
+            }
+            // a column's maxima are few: most slots of a wave hold none
+            if (__builtin_amdgcn_ballot_w64(x[0] == mx[0]) | __builtin_amdgcn_ballot_w64(x[1] == mx[1]) |
+                __builtin_amdgcn_ballot_w64(x[2] == mx[2]) | __builtin_amdgcn_ballot_w64(x[3] == mx[3])) {
+#pragma unroll
+                for (int u = 0; u < 4; u++) o[u] += x[u] == mx[u] ? sh[u] : 0.0f;
             }
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, o), dr, off, soff, 0);
             // Wait states after the 16-byte store before anything may rewrite its data registers: without them a VALU
@@ -677,7 +720,7 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
         soff = 0;
 #pragma unroll
         for (int i = 1; i < kRegs; i++) {
-            if (i <= nfull) put(v[i], voff, soff);
+            if (strip_in(i, nfull)) put(v[i], voff, soff);
             soff += rstepB;
             asm volatile("" : "+s"(soff));
         }
