@@ -600,8 +600,7 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
                     __hip_atomic_store(mine + k * kStripCols + lane, own[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // performed where the XCDs are coherent, before the arrival
             if (lane == 0) {
-                __hip_atomic_fetch_add(arrive, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                int got = __hip_atomic_load(arrive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                int got = __hip_atomic_fetch_add(arrive, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
                 for (int k = 0; k < spin && got < parts; k++) {
                     __builtin_amdgcn_s_sleep(4);
                     got = __hip_atomic_load(arrive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -611,12 +610,21 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
         }
         __syncthreads();
         if (flag) {
-            if (tid < kStripCols)
-                for (int p = 0; p < parts; p++)
+            // one value a thread and pass, every load in flight at once (a thread that took its column's parts one after the
+            // other paid 1.1 us a part: 8192 x 64 in 16 parts: 26.4 us, so 11.3)
+            constexpr int kPer = kParts * 4 * kStripCols / kStripThreads;
+            const float *const all = stats + (long)strip * parts * (4 * kStripCols);
+            float got[kPer];
 #pragma unroll
-                    for (int k = 0; k < 4; k++)
-                        pstat[k][p][tid] = __hip_atomic_load(stats + ((long)strip * parts + p) * (4 * kStripCols) + k * kStripCols + tid,
-                                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            for (int j = 0; j < kPer; j++)
+                got[j] = tid + j * kStripThreads < parts * 4 * kStripCols
+                             ? __hip_atomic_load(all + tid + j * kStripThreads, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0f;
+#pragma unroll
+            for (int j = 0; j < kPer; j++) {
+                const int i = tid + j * kStripThreads;
+                pstat[i / kStripCols % 4][i / (4 * kStripCols)][i % kStripCols] = got[j];
+            }
+            __syncthreads();
         } else {
             // the same statistics from memory, slot for slot in the order their own workgroup takes them
             for (int p = 0; p < parts; p++) {
@@ -758,7 +766,10 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
 }
 
 // Parts per strip and rows per part: as few parts as hold the rows on chip, then more while the workgroups stay within one
-// per CU and each keeps 8 slots (512 rows: less leaves a workgroup nothing to overlap its fixed cost with).
+// per CU and each keeps 8 slots (512 rows). Two workgroups per CU: 4096 x 4096 34.7 us for 31.8, 3008 x 2048 19.9 for 18.4;
+// parts of 256 rows: 512 x 2048 9.3 us for 8.8, 1024 x 64 8.6 for 9.8. Against the three kernels this is faster at every
+// shape measured from 64 x 64 (6.1 us for 11.3) over 4096 x 64 (10.5 for 14.8), 2048 x 2048 (15.8 for 17.4), 16384 x 64 (13.9
+// for 14.5) and 16384 x 1024 (34.5 for 44.9) to 8192 x 4096, so they are left the shapes that do not fit.
 struct StripPlan {
     int parts, rows;
 };
