@@ -75,6 +75,9 @@ struct ah_device {
     float *chain_scratch = nullptr;
     // Split-K workspace of the f32 tiled contractions (counters, then partial tiles), set up by ah_open.
     void *splitk_ws = nullptr;
+    // Loss workspace of ah_softmax_ce (kSoftmaxWsFloats), after the split-K partial tiles in the same allocation: its kernels
+    // run in this handle's stream order.
+    float *softmax_ws = nullptr;
 };
 
 struct ah_graph {

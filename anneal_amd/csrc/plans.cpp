@@ -1290,13 +1290,9 @@ int ah_gemm_tune(ah_device *dev, const ah_gemm_desc *d, int32_t iterations, int3
 
 int ah_softmax_ce(ah_device *dev, const float *z, const int32_t *labels, int32_t B, int32_t C, float *dz, float *loss) {
     if (!dev || !z || !labels || !dz || !loss || B <= 0 || C <= 0) return set_error(AH_ERR_INVALID, "ah_softmax_ce: bad argument");
-    float *rl = nullptr;
-    AH_HIP(hipMalloc(&rl, (size_t)B * 4));
-    float a = (float)(-1.0 / (double)B);
-    hipError_t e = softmax_ce(z, labels, B, C, a, dz, rl, dev->stream);
-    if (e == hipSuccess) e = sum_scale(rl, B, a, loss, dev->stream);
+    const float a = (float)(-1.0 / (double)B);
+    hipError_t e = softmax_ce(z, labels, B, C, a, dz, nullptr, dev->stream, loss, dev->softmax_ws);
     if (e == hipSuccess) e = hipStreamSynchronize(dev->stream);
-    hipFree(rl);
     if (e != hipSuccess) return fail_hip(e, "ah_softmax_ce");
     return AH_OK;
 }

@@ -23,9 +23,11 @@ constexpr int kSoftmaxColsMaxBlocks = 256;
 int softmax_ce_cols_blocks(int B);
 hipError_t softmax_ce_cols(const float *z, const int32_t *labels, int B, int C, float a, float *dz, float *rowloss,
                            float *part, hipStream_t s);
+// rowloss (each row's log-probability of its label) and loss (a * their sum) are both optional; loss takes ws,
+// kSoftmaxWsFloats floats, zero before the first call; its counters are left zero.
+constexpr int kSoftmaxWsFloats = 2048;
 hipError_t softmax_ce(const float *z, const int32_t *labels, int B, int C, float a, float *dz, float *rowloss,
-                      hipStream_t s);
-hipError_t sum_scale(const float *v, int n, float a, float *out, hipStream_t s);
+                      hipStream_t s, float *loss = nullptr, float *ws = nullptr);
 hipError_t mse_finalize(const float *acc, float scale, float *out, hipStream_t s);
 
 struct TailSeg {

@@ -82,13 +82,178 @@ __global__ __launch_bounds__(256) void colsum_kernel(const float *G, int M, int 
 
 // ── softmax cross-entropy ───────────────────────────────────────────────────
 // loss = Sum(onehot * logp) * a,  a = f32(-1/B); see the oracle's ora_softmax_ce for the op list.
-__global__ __launch_bounds__(256) void softmax_ce_kernel(const float *z, const int32_t *labels, int B, int C,
-                                                          float a, float *dz, float *rowloss) {
-    int row = blockIdx.x * 4 + (threadIdx.x >> 6);
-    int lane = threadIdx.x & 63;
-    if (row >= B) return;
-    const float rl = softmax_ce_row(z + (long)row * C, labels[row], C, a, dz + (long)row * C, lane);
-    if (lane == 0) rowloss[row] = rl;
+// The mean loss of a softmax-CE kernel without a second launch: `mine` is a workgroup's sum of its rows' terms (thread 0).
+// Workgroup b stores it to slot b; the last to arrive adds the slots, thread t slots t, t + blockDim, ..., then the threads in
+// order, so the result does not depend on timing. Arrivals at one counter queue up (256 of them: 4096 x 512 21.0 us a call, so 19.3; without the loss 16.9), so past 16
+// workgroups each of 16 counters takes a sixteenth of them, and its last arrival goes on to the root's. ws: the root counter,
+// the 16 others (a 128-byte line each, all zero before and after), the slots. red: one float a wave.
+constexpr int kSmGroups = 16, kSmLine = 32, kSmSlots = (1 + kSmGroups) * kSmLine;
+__device__ __forceinline__ void softmax_loss_fold(float mine, float a, float *loss, float *ws, float *red) {
+    __shared__ int last;
+    const int n = gridDim.x;
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(ws + kSmSlots + blockIdx.x, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int g = blockIdx.x % kSmGroups;
+        int *const group = (int *)ws + (1 + g) * kSmLine;
+        last = 1;
+        if (n > kSmGroups) {
+            last = ticket_take_atomic_partials(group) == (n - g + kSmGroups - 1) / kSmGroups - 1;
+            if (last) __hip_atomic_store(group, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (last) last = ticket_take_atomic_partials((int *)ws) == min(n, kSmGroups) - 1;
+    }
+    __syncthreads();
+    if (!last) return;
+    float v = 0.0f;
+    for (int i = threadIdx.x; i < n; i += blockDim.x)
+        v += __hip_atomic_load(ws + kSmSlots + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    v = wave_sum(v);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < (int)blockDim.x / 64; w++) v += red[w];
+        loss[0] = v * a;
+        __hip_atomic_store((int *)ws, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+// Softmax-CE of rows of up to 64 * VPR logits, a wave a row, the row held in registers between its three wave reductions
+// (softmax_ce_row reads it from memory four times) and the wave's next row loading meanwhile. Bound by those reductions'
+// latency: up to 256 workgroups of 1 to 16 waves, so that a wave has more than one row only past 4096 rows and the loss takes
+// at most 256 arrivals (128 workgroups: 16384 x 1024 47.5 us a call for 39.5). Against four reads of the row and a second
+// launch for the loss: 4096 x 512 26.1 -> 19.3 us a call, 16384 x 1024 82.0 -> 39.5 (134 MB, 25 us at the copy rate).
+constexpr int kSmWaves = 16, kSmBlocks = 256;
+template <int VPR>
+__global__ __launch_bounds__(64 * kSmWaves) void softmax_ce_kernel(const float *z, const int32_t *labels, int B, int C,
+                                                                   float a, float *dz, float *rowloss, float *loss, float *ws) {
+    __shared__ float red[kSmWaves];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6, step = gridDim.x * waves;
+    int row = blockIdx.x * waves + wave;
+    float nv[VPR], sum = 0.0f, col[VPR] = {};   // col: column sums, not asked for here
+    if (row < B) softmax_ce_row_load<VPR>(z + (long)row * C, C, lane, nv);
+    for (; row < B; row += step) {
+        float v[VPR];
+#pragma unroll
+        for (int j = 0; j < VPR; j++) v[j] = nv[j];
+        if (row + step < B) softmax_ce_row_load<VPR>(z + (long)(row + step) * C, C, lane, nv);
+        const float rl = softmax_ce_row_regs<VPR>(v, z + (long)row * C, labels[row], C, a, dz + (long)row * C, lane, col);
+        if (rowloss && lane == 0) rowloss[row] = rl;
+        sum += rl;
+    }
+    if (!loss) return;
+    if (lane == 0) red[wave] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        for (int w = 1; w < waves; w++) sum += red[w];
+    __syncthreads();   // red is reused by the fold
+    softmax_loss_fold(sum, a, loss, ws, red);
+}
+
+// Rows of more than 1024 and up to 512 * VPR logits: a workgroup of 8 waves a row, held in registers. Bound by the three
+// workgroup reductions and, with many rows, by memory. One wave a row from memory: 1 x 8192 77.4 us a call, 2000 x
+// 8192 164.7; so 17.8 and 40.2.
+constexpr int kSmWideThreads = 512, kSmWideWaves = kSmWideThreads / 64;
+template <int VPR>
+__global__ __launch_bounds__(kSmWideThreads) void softmax_ce_wide_kernel(const float *z, const int32_t *labels, int B, int C,
+                                                                         float a, float *dz, float *rowloss, float *loss, float *ws) {
+#pragma clang fp contract(off)   // each reference op rounds on its own, as in softmax_ce_row
+    __shared__ float red[4][kSmWideWaves];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    auto load = [&](int row, float (&v)[VPR]) {
+#pragma unroll
+        for (int j = 0; j < VPR; j++) {
+            const int c = tid + kSmWideThreads * j;
+            v[j] = c < C ? z[(long)row * C + c] : -FLT_MAX;
+        }
+    };
+    auto fold = [&](int k) {   // the waves' sums in order, the same in every thread
+        float r = red[k][0];
+#pragma unroll
+        for (int w = 1; w < kSmWideWaves; w++) r += red[k][w];
+        return r;
+    };
+    float nv[VPR], total = 0.0f;
+    int row = blockIdx.x;
+    load(row, nv);   // the grid has no more workgroups than rows
+    for (; row < B; row += gridDim.x) {
+        float v[VPR], e[VPR];
+#pragma unroll
+        for (int j = 0; j < VPR; j++) v[j] = nv[j];
+        if (row + (int)gridDim.x < B) load(row + gridDim.x, nv);
+        const int lab = labels[row];
+        const bool in = lab >= 0 && lab < C;
+        const float zl = in ? z[(long)row * C + lab] : 0.0f;
+        float m = -FLT_MAX;
+#pragma unroll
+        for (int j = 0; j < VPR; j++) m = fmaxf(m, v[j]);
+        m = wave_max(m);
+        if (lane == 0) red[0][wave] = m;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < kSmWideWaves; w++) m = fmaxf(m, red[0][w]);
+        float tie = 0.0f, s = 0.0f;
+#pragma unroll
+        for (int j = 0; j < VPR; j++) {
+            e[j] = exp2f((v[j] - m) * AH_INV_LN2);
+            if (tid + kSmWideThreads * j < C) {
+                tie += v[j] == m ? 1.0f : 0.0f;
+                s += e[j];
+            }
+        }
+        tie = wave_sum(tie);
+        s = wave_sum(s);
+        if (lane == 0) {
+            red[1][wave] = tie;
+            red[2][wave] = s;
+        }
+        __syncthreads();
+        tie = fold(1);
+        s = fold(2);
+        const float ls = log2f(s) * AH_LN2;
+        const float rl = in ? ((zl - m) - ls) : 0.0f;
+        const float gls = in ? -a : 0.0f;
+        const float gs = (gls * AH_LN2) * (1.0f / (s * AH_LN2));
+        float gm = 0.0f;
+#pragma unroll
+        for (int j = 0; j < VPR; j++) {
+            const int c = tid + kSmWideThreads * j;
+            e[j] = (c == lab ? a : 0.0f) + ((gs * e[j]) * AH_LN2) * AH_INV_LN2;
+            if (c < C) gm += -e[j];
+        }
+        gm = wave_sum(gm);
+        if (lane == 0) red[3][wave] = gm;
+        __syncthreads();   // a wave at the next row's red[0] store has passed here, where all have read red[0]; so for the others
+        const float share = fold(3) * (1.0f / tie);
+#pragma unroll
+        for (int j = 0; j < VPR; j++) {
+            const int c = tid + kSmWideThreads * j;
+            if (c < C) dz[(long)row * C + c] = v[j] == m ? e[j] + share : e[j];
+        }
+        if (rowloss && tid == 0) rowloss[row] = rl;
+        total += rl;
+    }
+    if (!loss) return;
+    __syncthreads();   // red is reused by the fold
+    softmax_loss_fold(total, a, loss, ws, red[0]);
+}
+
+// Longer rows: a wave a row, from memory.
+__global__ __launch_bounds__(256) void softmax_ce_long_kernel(const float *z, const int32_t *labels, int B, int C,
+                                                              float a, float *dz, float *rowloss, float *loss, float *ws) {
+    __shared__ float red[4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float sum = 0.0f;
+    for (int row = blockIdx.x * 4 + wave; row < B; row += gridDim.x * 4) {
+        const float rl = softmax_ce_row(z + (long)row * C, labels[row], C, a, dz + (long)row * C, lane);
+        if (rowloss && lane == 0) rowloss[row] = rl;
+        sum += rl;
+    }
+    if (!loss) return;
+    if (lane == 0) red[wave] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) sum = ((red[0] + red[1]) + red[2]) + red[3];
+    __syncthreads();
+    softmax_loss_fold(sum, a, loss, ws, red);
 }
 
 // Softmax-CE with the logit gradient's column sums (the output bias gradient) fused in: each wave
@@ -98,7 +263,6 @@ __global__ __launch_bounds__(256) void softmax_ce_kernel(const float *z, const i
 // tail), so the result does not depend on timing. With 16 waves per block and up to 256 blocks, a batch
 // of up to 4096 rows gives every wave one row: the row's three dependent wave reductions then overlap
 // across waves instead of running back to back in one.
-constexpr int kSmWaves = 16;
 template <int VPR>
 __global__ __launch_bounds__(64 * kSmWaves) void softmax_ce_cols_kernel(const float *z, const int32_t *labels, int B, int C,
                                                                         float a, float *dz, float *rowloss, float *part) {
@@ -129,20 +293,6 @@ __global__ __launch_bounds__(64 * kSmWaves) void softmax_ce_cols_kernel(const fl
         for (int w = 1; w < kSmWaves; w++) acc += red[w][c];
         part[(long)blockIdx.x * C + c] = acc;
     }
-}
-
-// out[0] = (Sum_i v[i]) * a   (single block, fixed-order tree)
-__global__ __launch_bounds__(256) void sum_scale_kernel(const float *v, int n, float a, float *out) {
-    __shared__ float red[256];
-    float acc = 0.0f;
-    for (int i = threadIdx.x; i < n; i += 256) acc += v[i];
-    red[threadIdx.x] = acc;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[0] = red[0] * a;
 }
 
 // MSE loss finalize: f16 reduce narrowing f16(acc) (codegen/lower.go:712) then * scale in f32.
@@ -975,9 +1125,31 @@ hipError_t colsum_add(const float *G, int M, int N, long ld, float *out, hipStre
     return hipGetLastError();
 }
 hipError_t softmax_ce(const float *z, const int32_t *labels, int B, int C, float a, float *dz, float *rowloss,
-                      hipStream_t s) {
+                      hipStream_t s, float *loss, float *ws) {
     if (B <= 0) return hipSuccess;
-    hipLaunchKernelGGL(softmax_ce_kernel, dim3((B + 3) / 4), dim3(256), 0, s, z, labels, B, C, a, dz, rowloss);
+    if (loss && !ws) return hipErrorInvalidValue;
+    static_assert(kSoftmaxWsFloats >= kSmSlots + 2 * kSmBlocks, "one slot a workgroup");
+    if (C <= 1024) {
+        const int waves = std::min(kSmWaves, (B + kSmBlocks - 1) / kSmBlocks);
+        const dim3 grid(std::min(kSmBlocks, (B + waves - 1) / waves)), block(64 * waves);
+#define AH_SM(n) hipLaunchKernelGGL(softmax_ce_kernel<n>, grid, block, 0, s, z, labels, B, C, a, dz, rowloss, loss, ws)
+        if (C <= 64) AH_SM(1);
+        else if (C <= 128) AH_SM(2);
+        else if (C <= 256) AH_SM(4);
+        else if (C <= 512) AH_SM(8);
+        else AH_SM(16);
+#undef AH_SM
+    } else if (C <= 16 * kSmWideThreads) {
+        const dim3 grid(std::min(2 * kSmBlocks, B)), block(kSmWideThreads);
+#define AH_SM(n) hipLaunchKernelGGL(softmax_ce_wide_kernel<n>, grid, block, 0, s, z, labels, B, C, a, dz, rowloss, loss, ws)
+        if (C <= 4 * kSmWideThreads) AH_SM(4);
+        else if (C <= 8 * kSmWideThreads) AH_SM(8);
+        else AH_SM(16);
+#undef AH_SM
+    } else {
+        hipLaunchKernelGGL(softmax_ce_long_kernel, dim3(loss ? std::min(2 * kSmBlocks, (B + 3) / 4) : (B + 3) / 4), dim3(256), 0, s, z,
+                           labels, B, C, a, dz, rowloss, loss, ws);
+    }
     return hipGetLastError();
 }
 int softmax_ce_cols_blocks(int B) {
@@ -994,10 +1166,6 @@ hipError_t softmax_ce_cols(const float *z, const int32_t *labels, int B, int C, 
     else if (C <= 512) hipLaunchKernelGGL(softmax_ce_cols_kernel<8>, grid, block, 0, s, z, labels, B, C, a, dz, rowloss, part);
     else if (C <= kSoftmaxColsMaxC) hipLaunchKernelGGL(softmax_ce_cols_kernel<16>, grid, block, 0, s, z, labels, B, C, a, dz, rowloss, part);
     else return hipErrorInvalidValue;
-    return hipGetLastError();
-}
-hipError_t sum_scale(const float *v, int n, float a, float *out, hipStream_t s) {
-    hipLaunchKernelGGL(sum_scale_kernel, dim3(1), dim3(256), 0, s, v, n, a, out);
     return hipGetLastError();
 }
 hipError_t mse_finalize(const float *acc, float scale, float *out, hipStream_t s) {

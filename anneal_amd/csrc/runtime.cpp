@@ -120,8 +120,13 @@ int ah_open(int ordinal, ah_device **out) {
     }
     {   // split-K counters start at zero; the kernels leave them at zero
         const size_t sync_bytes = (size_t)kSplitKMaxTiles * 2 * sizeof(int);
-        e = hipMalloc(&d->splitk_ws, sync_bytes + (size_t)kSplitKPartFloats * sizeof(float));
+        const size_t part_bytes = (size_t)kSplitKPartFloats * sizeof(float);
+        e = hipMalloc(&d->splitk_ws, sync_bytes + part_bytes + kSoftmaxWsFloats * sizeof(float));
         if (e == hipSuccess) e = hipMemset(d->splitk_ws, 0, sync_bytes);
+        if (e == hipSuccess) {
+            d->softmax_ws = (float *)((char *)d->splitk_ws + sync_bytes + part_bytes);
+            e = hipMemset(d->softmax_ws, 0, kSoftmaxWsFloats * sizeof(float));   // its counter, likewise
+        }
         if (e != hipSuccess) {
             if (d->splitk_ws) hipFree(d->splitk_ws);
             hipStreamDestroy(d->stream);

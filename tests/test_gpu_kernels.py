@@ -136,6 +136,41 @@ def test_softmax_ce_kernel(dev, B, C):
     assert abs(dloss.read()[0] - wl) <= 1e-5 * max(1.0, abs(wl))
 
 
+@pytest.mark.parametrize("B,C", [(1, 2), (255, 64), (257, 65), (300, 128), (4097, 129), (8200, 256), (5, 513), (9, 1024),
+                                 (1, 1025), (700, 2048), (3, 2049), (513, 4097), (2, 8192), (3, 8193)])
+def test_softmax_ce_edges(dev, B, C):
+    """Edges of the rows' kernels (a wave a row to 1024 logits, a workgroup to 8192, then a wave from memory; several rows
+    a wave or workgroup), called twice (the second call reads the workspace the first one left), and the item's row terms.
+    dz and the loss are sums of up to C terms in f32 against float64: at most 12 tree levels and 32 terms a lane, each
+    rounding 2^-24, over an exponential good to a few ulp: 1e-5 of the largest leaves a factor of 3."""
+    rng = np.random.default_rng(B * 8209 + C)
+    z = (rng.standard_normal((B, C)) * 3).astype(np.float32)
+    z[B // 2, : min(C, 3)] = z[B // 2].max() + 1.0   # a tied maximum
+    lab = rng.integers(0, C, B).astype(np.int32)
+    lab[0] = C                                       # no such column: no term, no gradient
+    x = z.astype(np.float64)
+    m = x.max(1, keepdims=True)
+    e = np.exp(x - m)
+    logp = x - m - np.log(e.sum(1, keepdims=True))
+    inside = lab < C
+    rows = np.where(inside, logp[np.arange(B), np.minimum(lab, C - 1)], 0.0)
+    P = e / e.sum(1, keepdims=True)
+    d = P.copy()
+    d[np.arange(B)[inside], lab[inside]] -= 1.0      # the max's own gradient is the sum of the others', zero up to rounding
+    d[~inside] = 0.0
+    dz_, dl_, dd, dloss = dev.buffer(z), dev.buffer(lab, L.AH_I32), dev.buffer(B * C), dev.buffer(1)
+    for _ in range(2):
+        dev.softmax_ce(dz_, dl_, B, C, dd, dloss)
+        got = dd.read().reshape(B, C).astype(np.float64) * B
+        assert np.abs(got - d).max() <= 1e-5
+        want = -rows.sum() / B
+        assert abs(dloss.read()[0] - want) <= 1e-5 * max(1.0, abs(want))
+    bufs = [Buffer(12, B * C, [B, C]), Buffer(11, B * C, [B, C]), Buffer(2, B, [B], L.AH_I32), Buffer(13, B, [B])]
+    out = Executor(dev).run([ExecItem(f"tmpl:softmax_ce;B={B};C={C}", bufs)], {11: z.ravel(), 2: lab.view(np.float32)})
+    assert np.array_equal(out[12].view(np.uint32), dd.read().view(np.uint32).ravel())
+    assert np.abs(out[13] - rows).max() <= 1e-5 * max(1.0, np.abs(rows).max())
+
+
 # (4096, 256), (8192, 64) and (8192, 528): the column-strip kernel that holds X on chip; the others: the
 # three-kernel chain
 @pytest.mark.parametrize("R,Cc,grow", [(64, 32, False), (257, 260, False), (1024, 512, False), (4096, 256, False),
