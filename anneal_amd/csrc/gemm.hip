@@ -333,7 +333,7 @@ __global__ __launch_bounds__(kThreads * KG) void gemm_kernel(GemmDesc d) {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's partial has landed
         }
         __syncthreads();
-        if (threadIdx.x == 0) ticket = ticket_take(count);
+        if (threadIdx.x == 0) ticket = ticket_take_atomic_partials(count);
         __syncthreads();
         if (ticket != nsplit - 1 || kg > 0) return;
         // every other split stored its partial before taking its ticket; add them in split order, one

@@ -51,7 +51,7 @@ struct G16Split {
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's partial has landed
         __syncthreads();
-        if (threadIdx.x == 0) *ticket = ticket_take(count);
+        if (threadIdx.x == 0) *ticket = ticket_take_atomic_partials(count);
         __syncthreads();
         if (*ticket != nsplit - 1) return false;
         // every other split stored its partial before taking its ticket; add them in split order,

@@ -244,7 +244,7 @@ __global__ __launch_bounds__(256) void gemm32d_kernel(GemmDesc d) {
     if (nsplit > 1) {
         // The register-staged kernel's split-K finish: every split stores its partial with 16-byte sc1
         // buffer stores (written through, coherent across the XCDs' L2s), waits for them, and takes a
-        // ticket from the tile's arrival counter (acquire-release); the split drawing the last ticket adds
+        // ticket from the tile's arrival counter; the split drawing the last ticket adds
         // all partials in split order (its own from registers), resets the counter and runs the epilogue.
         // Partial layout: 16-byte chunk c of thread t at byte 16 * (c * 256 + t) of its split.
         constexpr int NC = FM * FM * 4, PART = NC * 256 * 16, SC1 = 16;
@@ -268,7 +268,7 @@ __global__ __launch_bounds__(256) void gemm32d_kernel(GemmDesc d) {
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        if (tid == 0) ticket = ticket_take(count);
+        if (tid == 0) ticket = ticket_take_atomic_partials(count);
         __syncthreads();
         if (ticket != nsplit - 1) return;
 #pragma unroll
