@@ -1,10 +1,11 @@
 // rowops.hip — row reductions, loss-gradient epilogues and small elementwise kernels (gfx950).
 //
-// Softmax cross-entropy: one wave64 per row, shuffle reductions for the row max, the tie count and
-// the exp-sum; the backward follows the reference's op-by-op rules so the gradient through the row
+// Softmax cross-entropy: one wave64 per row (a workgroup past 1024 logits), shuffle reductions for the row
+// max, the tie count and the exp-sum; the backward follows the reference's op-by-op rules so the gradient through the row
 // max (tensor/gradient_ruleset.go:307-320, no stop-gradient in the reference) is reproduced.
 //
-// Movement chain (config 5): two streaming passes over X in its stored [R, Cc] layout. A Y-row is an
+// Movement chain (config 5): column strips of X held on chip between one read of X and one write of dX; where
+// they do not fit, two streaming passes over X in its stored [R, Cc] layout. A Y-row is an
 // X-column, so lanes own columns and walk rows: every wave load is a contiguous 1 KiB row segment
 // (float4 per lane) and no transpose is ever materialized. Pass 1 keeps online (max, tie count,
 // sum e, sum e^2) per column; a per-column finalize folds the row chunks and evaluates the
@@ -1219,9 +1220,9 @@ hipError_t chain_step(const float *X, const float *g, int R, int Cc, float *work
 // address until the process ends; host code must use the address hipGetSymbolAddress returned for the
 // current device, never the array's name (which is only a host-side stand-in).
 // The chain writes every workspace entry before reading it (chain_stats fills every chunk partial,
-// chain_finalize every coefficient and loss partial; the resident path every strip's loss sum), except
-// the resident path's arrival counter in word 0: static storage starts at zero and every call leaves
-// it zero, so nothing needs clearing between calls.
+// chain_finalize every coefficient and loss partial; the strip kernel every strip's loss sum and every
+// part's statistics), except the strip kernel's counters (word 0, and the strips' after the arrays): static
+// storage starts at zero and every call leaves them zero, so nothing needs clearing between calls.
 namespace ah {
 namespace {
 constexpr long kChainScratchFloats = 1L << 22;   // 16 MiB: R x Cc up to 16320 x 4096 (config 5, 8192 x 4096, needs 2.13M floats)

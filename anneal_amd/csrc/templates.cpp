@@ -24,7 +24,8 @@
 //   conv2d_bwd_b  data0 db [Co], data1 g [N,Co,H,H].
 //   sgd         data0 p' [n], data1 p, data2 g; p' = p - lr*(scale*g)  (Parameter.SGDStep, nn.go:69-76).
 //   mse_loss    data0 loss [1], data1 per-wave partials [parts]; loss = f16(sum) * scale.
-//   chain       data0 dX [R,Cc], data1 X [R,Cc], data2 g [Cc]; side data3 dg [Cc], data4 loss [1].
+//   chain       data0 dX [R,Cc], data1 X [R,Cc], data2 g [Cc]; side data3 dg [Cc], data4 loss [1];
+//               spin=n: polls before a workgroup takes other parts' statistics itself (the result does not depend on it).
 #include <math.h>
 #include <stdlib.h>
 #include <string.h>

@@ -143,7 +143,7 @@ def mlp3_f16(B, D0, D1, D2, D3):
 
 def chain(R, Cc):
     """Config 5: Y = Shrink(Pad(Permute(X, (1, 0)))), row softmax, RMS normalisation times g, Sum, and the
-    backward into X and g, as one chain item (its three kernels share a workspace)."""
+    backward into X and g, as one chain item."""
     lv = dict(X=1, g=2)
     items = [ExecItem(f"tmpl:chain;R={R};Cc={Cc}", [_buf(10, (R, Cc)), _buf(1, (R, Cc)), _buf(2, (Cc,)),
                                                      _buf(11, (Cc,)), _buf(12, (1,))])]

@@ -285,7 +285,7 @@ int ah_beam_apply(const char *key, char *out, int64_t cap, int64_t *needed);
 int ah_beam_cache(const char *path, int32_t save);
 void ah_beam_reset(void);   /* BeamCacheReset (beam.go:213) */
 
-/* Softmax cross-entropy forward+backward composed from reference ops (one wave64 per row):
+/* Softmax cross-entropy forward+backward composed from reference ops, one kernel:
  * m=Max, zs=z-m, e=Exp(zs), s=Sum e, logp=zs-Log(s), loss=Sum(onehot*logp)*(-1/B); dz includes the
  * row-max path with its tie split (tensor/gradient_ruleset.go:307-320). */
 int ah_softmax_ce(ah_device *dev, const float *z, const int32_t *labels, int32_t B, int32_t C, float *dz,
@@ -298,9 +298,9 @@ int ah_chain_step(ah_device *dev, const float *X, const float *g, int32_t R, int
 /* ah_chain_step without allocation. No counterpart in the reference: it is for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops). The chain's workspace is a
  * file-scope device array of 2^22 floats (16 MiB per GPU, held until the process ends), so
- * 64 + max(ceil(R/64)*Cc*4 + Cc*8 + ceil(Cc/16), Cc/16) must not exceed 2^22 (config 5, 8192 x 4096, needs 2.13M);
- * larger shapes fail with AH_ERR_INVALID. Asynchronous: the chain kernels (one at R = 8192, else three) are enqueued on the device
- * stream and the call returns (ah_sync waits). Every call on one GPU shares that GPU's workspace, so
+ * 64 + ceil(R/64)*Cc*4 + Cc*8 + ceil(Cc/16) must not exceed 2^22 (config 5, 8192 x 4096, needs 2.13M);
+ * larger shapes fail with AH_ERR_INVALID. Asynchronous: the chain's kernel (three where X does
+ * not fit on chip) is enqueued on the device stream and the call returns (ah_sync waits). Every call on one GPU shares that GPU's workspace, so
  * calls that overlap on one GPU (several device handles or host threads) race. */
 int ah_chain_step_noalloc(ah_device *dev, const float *X, const float *g, int32_t R, int32_t Cc, float *dX,
                           float *dg, float *loss);
