@@ -544,9 +544,9 @@ __device__ __forceinline__ float strip_tree_sum(float v) {
     return v + __shfl_xor(v, 32, 64);
 }
 
-// A thread's running statistics of its four columns: the reference mt its exponentials are taken against, sum e, sum e^2
-// and the exact running max. An element more than 2^60 above mt (where e^2 could overflow) first moves the reference to
-// itself. The elements equal to the max are counted afterwards, and only where a lane met its running max again (a bit of
+// A thread's running statistics of its four columns: the reference mt its exponentials are taken against (finite: -FLT_MAX
+// or above, so that an entry of -inf adds exp2(-inf) = 0), sum e, sum e^2 and the exact running max, from -FLT_MAX. An
+// element more than 2^60 above mt (where e^2 could overflow) first moves the reference to itself. The elements equal to the max are counted afterwards, and only where a lane met its running max again (a bit of
 // `tie`, kept in scalar registers): counting them as they land took 5 of 17 vector operations per element, in a kernel whose
 // vector work shows (8192 x 4096: 67.3 us with the count, 59.1 us without any statistics).
 struct StripStat {
@@ -591,11 +591,11 @@ struct StripStat {
                      "+v"(sq[3]), "+v"(mr[0]), "+v"(mr[1]), "+v"(mr[2]), "+v"(mr[3]));
     }
     // the elements equal to the thread's max, counted over each(f) (f is called with every element of the thread) where any
-    // lane of the wave may have more than one; some: the thread has an element at all
+    // lane of the wave may have more than one, or one of -FLT_MAX; else one set the max, or none did (-inf only, no element)
     template <class Each>
-    __device__ __forceinline__ void count(bool some, float (&cnt)[4], Each &&each) const {
+    __device__ __forceinline__ void count(float (&cnt)[4], Each &&each) const {
 #pragma unroll
-        for (int u = 0; u < 4; u++) cnt[u] = some ? 1.0f : 0.0f;
+        for (int u = 0; u < 4; u++) cnt[u] = mr[u] > -FLT_MAX ? 1.0f : 0.0f;
         if (tie == 0) return;
 #pragma unroll
         for (int u = 0; u < 4; u++) cnt[u] = 0.0f;
@@ -704,7 +704,7 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
     {
         float ref[4];
 #pragma unroll
-        for (int u = 0; u < 4; u++) ref[u] = ok0 ? v[0][u] : -FLT_MAX;
+        for (int u = 0; u < 4; u++) ref[u] = ok0 ? fmaxf(-FLT_MAX, v[0][u]) : -FLT_MAX;
 #pragma unroll
         for (int i = 1; i < kProv; i++)
             if (strip_in(i, nfull))
@@ -726,7 +726,7 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
         }
     }
     float cnt[4];
-    st.count(colok && (nfull > 0 || ok0), cnt, [&](auto &&f) {
+    st.count(cnt, [&](auto &&f) {
         if (ok0) f(v[0]);
 #pragma unroll
         for (int i = 1; i < kRegs; i++)
@@ -786,7 +786,7 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
                 const floatx4 x0 = pok ? *(const floatx4 *)(px + (long)r0 * Cc) : (floatx4){};
                 float ref[4];
 #pragma unroll
-                for (int u = 0; u < 4; u++) ref[u] = pok ? x0[u] : -FLT_MAX;
+                for (int u = 0; u < 4; u++) ref[u] = pok ? fmaxf(-FLT_MAX, x0[u]) : -FLT_MAX;
                 for (int i = 1; i < kProv && i <= pf; i++) {
                     const floatx4 x = at(i);
 #pragma unroll
@@ -796,7 +796,7 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
                 o.init(ref);
                 if (pok) o.push(x0);
                 for (int i = 1; i <= pf; i++) o.push(at(i));
-                o.count(colok && (pf > 0 || pok), cnt, [&](auto &&f) {
+                o.count(cnt, [&](auto &&f) {
                     if (pok) f(x0);
                     for (int i = 1; i <= pf; i++) f(at(i));
                 });

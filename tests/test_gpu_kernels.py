@@ -244,6 +244,46 @@ def test_chain_strip_edges(dev, R, Cc, spin):
             np.testing.assert_array_equal(out[k].view(np.uint32), v.view(np.uint32))
 
 
+# One slot (64 rows), a part of 512 rows, several parts, whole strips of one workgroup
+@pytest.mark.parametrize("R,Cc", [(1, 4), (64, 36), (1025, 100), (2049, 260), (3001, 2052), (4097, 64), (8192, 96), (9000, 8)])
+@pytest.mark.parametrize("spin", [-1, 0])
+def test_chain_infinite_entries(dev, R, Cc, spin):
+    """Entries of -inf (a mask) leave the chain finite, as exp2(-inf) = 0: a leading block, one row, a third of a column, the
+    first row of a thread, all but the last row, and beside -FLT_MAX only; a NaN or +inf makes its own column NaN and the
+    loss, no other column. Against the float64 closed form, with the bound of test_chain_strip_edges."""
+    rng = np.random.default_rng(R * 3 + Cc)
+    X = rng.standard_normal((R, Cc)).astype(np.float32)
+    ninf, low = np.float32(-np.inf), np.float32(-3.4028234663852886e38)
+    if R > 1:
+        X[R // 2, :] = ninf                                  # one row in all columns
+        X[:min(512, R - 1), 0] = ninf                        # a whole part where a part has 512 rows
+        X[: R // 3, 1] = ninf
+        X[:-1, 2] = ninf                                     # the last row alone is left
+        X[:, 3] = np.where(np.arange(R) % 3 == 0, low, ninf)  # nothing above -FLT_MAX
+    if Cc >= 32:
+        X[::64, 5] = ninf                                    # some lanes' first rows
+        X[R - 1, 6], X[0, 7] = np.nan, np.inf
+    g = (1 + 0.02 * rng.standard_normal(Cc)).astype(np.float32)
+    bufs = [Buffer(10, R * Cc, [R, Cc]), Buffer(1, R * Cc, [R, Cc]), Buffer(2, Cc, [Cc]), Buffer(11, Cc, [Cc]), Buffer(12, 1, [1])]
+    key = f"tmpl:chain;R={R};Cc={Cc}" + (f";spin={spin}" if spin >= 0 else "")
+    out = Executor(dev).run([ExecItem(key, bufs)], {1: X.ravel(), 2: g})
+    bad = ~(np.isfinite(X) | (X == ninf)).all(0)
+    got, x, g = out[10].reshape(R, Cc), X.astype(np.float64)[:, ~bad], g[~bad]
+    m = x.max(0)
+    e = np.exp(x - m)
+    S = e / e.sum(0)
+    T = np.sqrt((S * S).mean(0) + 1e-6)
+    dg = 1 / T
+    gS = g / T - S * (g * S.sum(0) / (R * T**3))
+    dX = S * (gS - (gS * S).sum(0))
+    assert np.all(np.abs(got[:, ~bad] - dX) <= 16 * 2.0**-23 * (S * g / T) + 4 * 2.0**-24 * (g / T) * (x == m) + 1e-30)
+    assert np.allclose(out[11][~bad], dg, rtol=1e-5)
+    if bad.any():
+        assert np.isnan(got[:, bad]).all() and np.isnan(out[11][bad]).all() and np.isnan(out[12][0])
+    else:
+        assert np.allclose(out[12][0], (g * dg).sum(), rtol=1e-5)
+
+
 F16_VARIANTS = list(range(1, 40))   # every gemm16 variant (gemm16_kernel.h Var<V>; 32-39 use 16x16x32 MFMAs)
 KGROUP_VARIANTS = (10, 11, 15, 25, 28, 31, 35, 36, 37, 38)   # variants that add two k-halves
 VARIANT_SHAPES = [
