@@ -916,7 +916,7 @@ struct ChainTrainer : ah_trainer {
         rc |= alloc(&X, (size_t)R * Cc); rc |= alloc(&g, Cc); rc |= alloc(&dX, (size_t)R * Cc);
         rc |= alloc(&dg, Cc); rc |= alloc(&work, chain_workspace_floats(R, Cc)); rc |= alloc(&loss, 1);
         if (rc) return AH_ERR_HIP;
-        AH_HIP(hipMemset(work, 0, sizeof(float) * chain_workspace_floats(R, Cc)));   // the arrival counter
+        AH_HIP(hipMemset(work, 0, sizeof(float) * chain_workspace_floats(R, Cc)));   // the counters
         return AH_OK;
     }
     int max_batch() const override { return R; }
@@ -1302,8 +1302,7 @@ int ah_chain_step(ah_device *dev, const float *X, const float *g, int32_t R, int
         return set_error(AH_ERR_INVALID, "ah_chain_step: bad argument (Cc must be a multiple of 4)");
     float *w = nullptr;
     AH_HIP(hipMalloc(&w, (size_t)chain_workspace_floats(R, Cc) * 4));
-    hipError_t e = hipMemsetAsync(w, 0, 256, dev->stream);   // the strip kernel's counters
-    if (e == hipSuccess) e = hipMemsetAsync(w + chain_array_floats(R, Cc), 0, (size_t)chain_sync_ints(Cc) * 4, dev->stream);
+    hipError_t e = hipMemsetAsync(w + chain_array_floats(R, Cc), 0, (size_t)chain_sync_ints(Cc) * 4, dev->stream);
     if (e == hipSuccess) e = chain_step(X, g, R, Cc, w, dX, dg, loss, dev->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(dev->stream);
     hipFree(w);
@@ -1320,7 +1319,7 @@ int ah_chain_step_noalloc(ah_device *dev, const float *X, const float *g, int32_
         return set_error(AH_ERR_INVALID, "ah_chain_step_noalloc: R=%d x Cc=%d needs %ld workspace floats, the maximum is %ld",
                          R, Cc, need, cap);
     if (!dev->chain_scratch) return set_error(AH_ERR_INVALID, "ah_chain_step_noalloc: device has no chain workspace");
-    AH_HIP(chain_step(X, g, R, Cc, dev->chain_scratch, dX, dg, loss, dev->stream, -1, (int *)(dev->chain_scratch + cap)));
+    AH_HIP(chain_step(X, g, R, Cc, dev->chain_scratch, dX, dg, loss, dev->stream, -1, dev->chain_sync));
     return AH_OK;
 }
 

@@ -56,20 +56,21 @@ struct TailArgs {
 };
 hipError_t step_tail(const TailArgs &t, hipStream_t s);
 
-// Workspace of the chain, in floats: its arrays (chain_array_floats, whose word 0 is a counter) and the arrival counters
-// of its strips after them (chain_sync_ints). Word 0 and the counters are zero before the first call and left zero.
+// Workspace of the chain, in floats: its arrays (chain_array_floats) and the strip kernel's counters after them
+// (chain_sync_ints), zero before the first call and left zero. chain_sync_max_ints: counters for any Cc the strips take.
 long chain_workspace_floats(int R, int Cc);
 long chain_array_floats(int R, int Cc);
 long chain_sync_ints(int Cc);
-// Capacity (floats) of the arrays in the file-scope chain workspace used by ah_chain_step_noalloc (the arrival counters
-// follow them), and its address on the device `ordinal` (the current device at the call).
+long chain_sync_max_ints();
+// Capacity (floats) of the arrays in the file-scope chain workspace used by ah_chain_step_noalloc, and its address on the
+// device `ordinal` (the current device at the call).
 long chain_scratch_floats();
 hipError_t chain_scratch_init(int ordinal, float **out);
 // True where the chain runs as one launch, each 32-column strip of X held on chip (one pass over HBM).
 bool chain_resident_fits(int R, int Cc);
 // The whole config-5 chain (phase -1: the strip kernel where it fits, else the three kernels below) or one of its three
 // kernels (phase 0 stats, 1 finalize, 2 gradient). work: chain_workspace_floats floats, or chain_array_floats with the
-// arrival counters at sync. spin: polls before a workgroup takes the other parts' statistics from X itself (-1: the default).
+// counters at sync. spin: polls before a workgroup takes the other parts' statistics from X itself (-1: the default).
 hipError_t chain_step(const float *X, const float *g, int R, int Cc, float *work, float *dX, float *dg, float *loss,
                       hipStream_t s, int phase = -1, int *sync = nullptr, int spin = -1);
 

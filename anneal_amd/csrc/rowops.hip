@@ -530,7 +530,7 @@ __global__ __launch_bounds__(256) void chain_grad_kernel(const float *X, int R, 
 constexpr int kStripThreads = 512, kStripWaves = kStripThreads / 64, kStripCols = 32, kStripRows = kStripThreads / 8;
 constexpr int kStripMaxRegs = 45, kStripMaxSlots = 64;   // float4 slots per thread in VGPRs; in all (19 in LDS: 152 KiB)
 constexpr int kStripMaxParts = 16, kStripMaxPartsFull = 4;   // parts whose statistics fit beside the held rows in LDS
-constexpr int kStripMaxStrips = 1024;                    // arrival counters of ah_chain_step_noalloc's workspace
+constexpr int kStripMaxStrips = 1024;                    // a handle's counters for ah_chain_step_noalloc
 constexpr int kStripSpin = 1 << 14;
 
 __device__ __forceinline__ float strip_tree_max(float v) {   // over the 8 lanes of a wave with equal lane & 7
@@ -1174,25 +1174,27 @@ hipError_t mse_finalize(const float *acc, float scale, float *out, hipStream_t s
     return hipGetLastError();
 }
 
-// Workspace: word 0 is the strip kernel's loss counter, zero before the first call and left zero by every call; from float
-// 64 either path's arrays; then the strips' arrival counters (likewise zero between calls; the three-kernel path touches
-// neither). ah_chain_step_noalloc, whose arrays serve every shape, keeps the arrival counters apart.
-constexpr long kChainHead = 64;
+// Workspace: from float 64 either path's arrays; then the strip kernel's counters, the loss's in a line of its own and two a
+// strip, zero before the first call and left zero by every call (the three-kernel path touches none). ah_chain_step_noalloc,
+// whose arrays serve every shape and every handle of a GPU, passes its handle's counters.
+constexpr long kChainHead = 64, kChainLossSync = 32;
 long chain_array_floats(int R, int Cc) {
     int nch = (R + kChainStatsRows - 1) / kChainStatsRows;
     const long three = (long)nch * Cc * 4 + (long)Cc * 8 + (Cc + kFinCols - 1) / kFinCols;
     const long strips = (Cc + kStripCols - 1) / kStripCols;   // their loss terms, and the parts' statistics
     return kChainHead + std::max(three, chain_resident_fits(R, Cc) ? strips * (1 + 4L * kStripCols * strip_plan(R, Cc).parts) : 0L);
 }
-long chain_sync_ints(int Cc) { return 2L * ((Cc + kStripCols - 1) / kStripCols); }
+long chain_sync_ints(int Cc) { return kChainLossSync + 2L * ((Cc + kStripCols - 1) / kStripCols); }
+long chain_sync_max_ints() { return chain_sync_ints(kStripMaxStrips * kStripCols); }
 long chain_workspace_floats(int R, int Cc) { return chain_array_floats(R, Cc) + chain_sync_ints(Cc); }
 
 hipError_t chain_step(const float *X, const float *g, int R, int Cc, float *work, float *dX, float *dg, float *loss,
                       hipStream_t s, int phase, int *sync, int spin) {
     if (Cc % 4 != 0 || R <= 0) return hipErrorInvalidValue;
-    if (phase < 0 && chain_resident_fits(R, Cc))
-        return chain_resident(X, g, R, Cc, work + kChainHead, sync ? sync : (int *)(work + chain_array_floats(R, Cc)), (int *)work, dX,
-                              dg, loss, spin < 0 ? kStripSpin : spin, s);
+    if (phase < 0 && chain_resident_fits(R, Cc)) {
+        if (!sync) sync = (int *)(work + chain_array_floats(R, Cc));
+        return chain_resident(X, g, R, Cc, work + kChainHead, sync + kChainLossSync, sync, dX, dg, loss, spin < 0 ? kStripSpin : spin, s);
+    }
     work += kChainHead;
     const int nch = (R + kChainStatsRows - 1) / kChainStatsRows;
     const int nfin = (Cc + kFinCols - 1) / kFinCols;
@@ -1221,13 +1223,14 @@ hipError_t chain_step(const float *X, const float *g, int R, int Cc, float *work
 // current device, never the array's name (which is only a host-side stand-in).
 // The chain writes every workspace entry before reading it (chain_stats fills every chunk partial,
 // chain_finalize every coefficient and loss partial; the strip kernel every strip's loss sum and every
-// part's statistics), except the strip kernel's counters (word 0, and the strips' after the arrays): static
-// storage starts at zero and every call leaves them zero, so nothing needs clearing between calls.
+// part's statistics), so nothing needs clearing between calls. The strip kernel's counters, which a launch
+// takes from zero back to zero, are not here but with each device handle: its launches run one after another
+// on its stream, whereas launches of two handles that overlap would leave shared counters wrong for good.
 namespace ah {
 namespace {
 constexpr long kChainScratchFloats = 1L << 22;   // 16 MiB: R x Cc up to 16320 x 4096 (config 5, 8192 x 4096, needs 2.13M floats)
 constexpr int kMaxDevices = 64;
-static __device__ __align__(256) float scratch[kChainScratchFloats + 2 * kStripMaxStrips];   // arrays, then arrival counters
+static __device__ __align__(256) float scratch[kChainScratchFloats];
 float *g_scratch_ptr[kMaxDevices];
 }  // namespace
 

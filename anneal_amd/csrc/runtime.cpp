@@ -121,11 +121,13 @@ int ah_open(int ordinal, ah_device **out) {
     {   // split-K counters start at zero; the kernels leave them at zero
         const size_t sync_bytes = (size_t)kSplitKMaxTiles * 2 * sizeof(int);
         const size_t part_bytes = (size_t)kSplitKPartFloats * sizeof(float);
-        e = hipMalloc(&d->splitk_ws, sync_bytes + part_bytes + kSoftmaxWsFloats * sizeof(float));
+        const size_t tail_bytes = kSoftmaxWsFloats * sizeof(float) + (size_t)chain_sync_max_ints() * sizeof(int);
+        e = hipMalloc(&d->splitk_ws, sync_bytes + part_bytes + tail_bytes);
         if (e == hipSuccess) e = hipMemset(d->splitk_ws, 0, sync_bytes);
         if (e == hipSuccess) {
             d->softmax_ws = (float *)((char *)d->splitk_ws + sync_bytes + part_bytes);
-            e = hipMemset(d->softmax_ws, 0, kSoftmaxWsFloats * sizeof(float));   // its counter, likewise
+            d->chain_sync = (int *)(d->softmax_ws + kSoftmaxWsFloats);
+            e = hipMemset(d->softmax_ws, 0, tail_bytes);   // the softmax's and the chain's counters, likewise
         }
         if (e != hipSuccess) {
             if (d->splitk_ws) hipFree(d->splitk_ws);

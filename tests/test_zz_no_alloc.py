@@ -42,3 +42,27 @@ def test_noalloc_rejects_shapes_beyond_the_workspace(dev):
         dev.chain_step_noalloc(bufs[0], bufs[1], R, Cc, bufs[2], bufs[3], bufs[4])
     for b in bufs:
         b.free()
+
+
+def test_overlapping_handles_leave_later_calls_right(dev):
+    """Two handles' calls that overlap share the workspace's arrays, so their own outputs are undefined; the strips' counters
+    are each handle's, so calls made alone afterwards are right on both (16 parts a strip here)."""
+    from anneal_amd.backend import Device
+    R, Cc = 8192, 64
+    rng = np.random.default_rng(3)
+    X, g = rng.standard_normal((R, Cc)).astype(np.float32), np.ones(Cc, np.float32)
+    with Device(0) as other:
+        want = _run(dev, dev.chain_step, X, g)
+        sets = [[d] + [d.buffer(X), d.buffer(g), d.buffer(R * Cc), d.buffer(Cc), d.buffer(1)] for d in (dev, other)]
+        for _ in range(100):
+            for d, *b in sets:
+                d.chain_step_noalloc(b[0], b[1], R, Cc, b[2], b[3], b[4])
+        for d, *b in sets:
+            d.sync()
+        for d, *b in sets:
+            for _ in range(2):
+                got = _run(d, d.chain_step_noalloc, X, g)
+                for x, y in zip(got, want):
+                    np.testing.assert_array_equal(x.view(np.uint32), y.view(np.uint32))
+            for x in b:
+                x.free()
