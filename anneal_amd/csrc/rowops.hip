@@ -521,8 +521,11 @@ __global__ __launch_bounds__(256) void chain_grad_kernel(const float *X, int R, 
 // 4096 with X in memory (49 us with X left in the Infinity Cache by the step before): 64-byte row segments use half of each
 // line, and only a neighbour on the same XCD can use the rest.
 //
-// Waiting for the other parts is bounded: a workgroup that has polled `spin` times takes the missing statistics from X
-// itself, in the same order, so the result is the same and nothing depends on the parts running together.
+// Waiting for the other parts is bounded: a workgroup that has polled `spin` times takes the missing parts' statistics from X
+// itself, in the same order, so the result is the same and nothing depends on the parts running together. That holds in place
+// too (dX over X, dg over g): the workgroup says that it reads before it looks again which parts are missing, and those wait
+// for it before they write (it runs, and itself waits for nobody meanwhile); dg is stored by the last part to leave, after
+// every part has read g.
 //
 // Thread t owns columns 4 (t & 7) .. + 3 of rows (t >> 3) + 64 i of its range: slot 0 the last, possibly partial 64 rows,
 // slots 1 .. nfull the whole ones. Every sum is a fixed tree (slots in order, then lanes by xor, waves in order, parts in
@@ -532,6 +535,10 @@ constexpr int kStripMaxRegs = 45, kStripMaxSlots = 64;   // float4 slots per thr
 constexpr int kStripMaxParts = 16, kStripMaxPartsFull = 4;   // parts whose statistics fit beside the held rows in LDS
 constexpr int kStripMaxStrips = 1024;                    // a handle's counters for ah_chain_step_noalloc
 constexpr int kStripSpin = 1 << 14;
+// A strip's arrival word: a bit for each part that has posted its statistics, and from bit 16 up the count of workgroups that
+// read other parts' rows of X. Polls for those readers (some us each) end after kStripReaderSpin, several seconds.
+constexpr int kStripReader = 1 << 16, kStripReaderSpin = 1 << 23;
+static_assert(kStripMaxParts <= 16, "a bit for each part below the readers' count");
 
 __device__ __forceinline__ float strip_tree_max(float v) {   // over the 8 lanes of a wave with equal lane & 7
     v = fmaxf(v, __shfl_xor(v, 8, 64));
@@ -645,12 +652,12 @@ __device__ __forceinline__ bool strip_in(int i, int nfull) {
 }
 
 // part_rows: rows per part (a multiple of 64, at most 64 * NS; the last part may have fewer). stats: parts * 128 floats a
-// strip. sync: two counters a strip, arrivals and departures, zero before and after.
+// strip. sync: two words a strip, arrivals and departures, zero before and after. in_place: dX or dg shares memory with X or g.
 template <int NS>
 __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float *X, int R, int Cc, int parts, int part_rows,
                                                                      const float *g, float *dX, float *dg, float *stats,
                                                                      int *sync, float *lossp, int *counter, float *loss,
-                                                                     int spin) {
+                                                                     int spin, int in_place) {
     constexpr int kRegs = NS < kStripMaxRegs ? NS : kStripMaxRegs, kLds = NS - kRegs, kProv = NS < 8 ? NS : 8;
     constexpr int kParts = NS > kStripMaxRegs ? kStripMaxPartsFull : kStripMaxParts;
     __shared__ __attribute__((aligned(1024))) floatx4 held[kLds > 0 ? kLds : 1][kStripThreads];
@@ -678,6 +685,7 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
     const long org = (long)rbeg * Cc + c0;
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void *)(X + org), (short)0, 0x7fffffff, 0x00020000);
     const __amdgpu_buffer_rsrc_t dr = __builtin_amdgcn_make_buffer_rsrc((void *)(dX + org), (short)0, 0x7fffffff, 0x00020000);
+    const float gi = tid < kStripCols && c0 + tid < Cc ? g[c0 + tid] : 0.0f;   // before this part arrives
     const int voff = colok ? (rl * Cc + 4 * q) * 4 : kOut, voff0 = ok0 ? (row0 * Cc + 4 * q) * 4 : kOut;
     const int rstepB = kStripRows * Cc * 4;
     // 1. the rows: register slots first (they are consumed first), then the LDS slots
@@ -740,6 +748,7 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
     __syncthreads();
     // 3. the part's column statistics, and the other parts'
     float own[4];
+    int reads = 0, leader = 1;   // thread 0: this part has said that it reads X; wave 0: this part stores dg
     if (tid < kStripCols) strip_fold(kStripWaves, [&](int k, int w) { return red[k][w][tid]; }, own);
     if (parts > 1) {
         float *const mine = stats + ((long)strip * parts + part) * (4 * kStripCols);
@@ -749,18 +758,23 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
 #pragma unroll
                 for (int k = 0; k < 4; k++)
                     __hip_atomic_store(mine + k * kStripCols + lane, own[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // performed where the XCDs are coherent, before the arrival
+            // performed where the XCDs are coherent, before the arrival; g has been read
+            asm volatile("s_waitcnt vmcnt(0)" :: "v"(gi) : "memory");
             if (lane == 0) {
-                int got = __hip_atomic_fetch_add(arrive, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
-                for (int k = 0; k < spin && got < parts; k++) {
+                const int all = (1 << parts) - 1;
+                int got = __hip_atomic_fetch_add(arrive, 1 << part, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) | 1 << part;
+                for (int k = 0; k < spin && (got & all) != all; k++) {
                     __builtin_amdgcn_s_sleep(4);
                     got = __hip_atomic_load(arrive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
-                flag = got >= parts;
+                reads = (got & all) != all;
+                if (reads) got = __hip_atomic_fetch_add(arrive, kStripReader, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                flag = all & ~got;
             }
         }
         __syncthreads();
-        if (flag) {
+        const int missing = flag;
+        if (missing == 0) {
             // one value a thread and pass, every load in flight at once (a thread that took its column's parts one after the
             // other paid 1.1 us a part: 8192 x 64 in 16 parts: 26.4 us, so 11.3)
             constexpr int kPer = kParts * 4 * kStripCols / kStripThreads;
@@ -777,8 +791,16 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
             }
             __syncthreads();
         } else {
-            // the same statistics from memory, slot for slot in the order their own workgroup takes them
+            // those that are there; the others from X, slot for slot in the order their own workgroup takes them
             for (int p = 0; p < parts; p++) {
+                if ((missing >> p & 1) == 0) {
+                    if (tid < kStripCols)
+#pragma unroll
+                        for (int k = 0; k < 4; k++)
+                            pstat[k][p][tid] = __hip_atomic_load(stats + (((long)strip * parts + p) * 4 + k) * kStripCols + tid,
+                                                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    continue;
+                }
                 const int pb = p * part_rows, pr = min(part_rows, R - pb), pf = (pr - 1) / kStripRows, r0 = pf * kStripRows + rl;
                 const bool pok = r0 < pr && colok;
                 const float *const px = X + (long)pb * Cc + col;
@@ -812,13 +834,21 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
             }
         }
         if (tid < kStripCols) strip_fold(parts, [&](int k, int p) { return pstat[k][p][tid]; }, own);
-        if (tid == 0) {   // the last part to leave (every one has arrived by then) clears the counters for the next launch
+        if (tid == 0) {
+            // every thread has its values of X by the fold's last barrier
+            if (reads) __hip_atomic_fetch_add(arrive, -kStripReader, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (in_place)
+                for (int k = 0; k < kStripReaderSpin && __hip_atomic_load(arrive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= kStripReader; k++)
+                    __builtin_amdgcn_s_sleep(4);
+            // the last part to leave (every one has arrived by then) clears the words for the next launch
             const int gone = __hip_atomic_fetch_add(arrive + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (gone == parts - 1) {
+            leader = gone == parts - 1;
+            if (leader) {
                 __hip_atomic_store(arrive, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 __hip_atomic_store(arrive + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
+        leader = __shfl(leader, 0, 64);   // to wave 0, whose lanes hold the columns
     }
     // 4. the column's scalars (chain_finalize's rules), the same in every part
     if (tid < kStripCols) {
@@ -832,7 +862,6 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
         const float qm = sqq * rR;
         const float T = sqrtf(qm + eps);
         const float r = 1.0f / T;
-        const float gi = live ? g[c] : 0.0f;
         const float gR = gi * sumS;
         const float gT = ((-gR) * r) * r;
         const float gu = gT * (1.0f / (2.0f * T));
@@ -848,7 +877,7 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
         coef[2][tid] = mm;
         coef[3][tid] = gm * (1.0f / t_);
         coef[4][tid] = live ? gi * (r * sumS) : 0.0f;
-        if (part == 0 && live) dg[c] = r * sumS;
+        if (leader && live) dg[c] = r * sumS;
     }
     __syncthreads();
     // 5. dX from the held rows
@@ -943,10 +972,10 @@ bool chain_resident_fits(int R, int Cc) {
 
 template <int NS>
 static void launch_strip(const float *X, const float *g, int R, int Cc, const StripPlan &p, float *stats, int *sync, float *lossp,
-                         int *counter, float *dX, float *dg, float *loss, int spin, hipStream_t s) {
+                         int *counter, float *dX, float *dg, float *loss, int spin, int in_place, hipStream_t s) {
     const int wgs = (Cc + kStripCols - 1) / kStripCols * p.parts;
     hipLaunchKernelGGL(chain_strip_kernel<NS>, dim3((wgs + 7) / 8 * 8), dim3(kStripThreads), 0, s, X, R, Cc, p.parts, p.rows, g,
-                       dX, dg, stats, sync, lossp, counter, loss, spin);
+                       dX, dg, stats, sync, lossp, counter, loss, spin, in_place);
 }
 
 hipError_t chain_resident(const float *X, const float *g, int R, int Cc, float *arrays, int *sync, int *counter, float *dX,
@@ -955,7 +984,13 @@ hipError_t chain_resident(const float *X, const float *g, int R, int Cc, float *
     const StripPlan p = strip_plan(R, Cc);
     const int strips = (Cc + kStripCols - 1) / kStripCols, slots = p.rows / kStripRows;
     float *lossp = arrays + (p.parts > 1 ? (long)strips * p.parts * 4 * kStripCols : 0);
-#define AH_STRIP(n) launch_strip<n>(X, g, R, Cc, p, arrays, sync, lossp, counter, dX, dg, loss, spin, s)
+    // dX or dg over X or g (over part of one: undefined)
+    const uintptr_t nx = (uintptr_t)R * Cc * 4, ng = (uintptr_t)Cc * 4;
+    auto meet = [](const float *a, uintptr_t na, const float *b, uintptr_t nb) {
+        return (uintptr_t)a < (uintptr_t)b + nb && (uintptr_t)b < (uintptr_t)a + na;
+    };
+    const int in_place = meet(dX, nx, X, nx) || meet(dg, ng, g, ng);
+#define AH_STRIP(n) launch_strip<n>(X, g, R, Cc, p, arrays, sync, lossp, counter, dX, dg, loss, spin, in_place, s)
     if (slots <= 4) AH_STRIP(4);
     else if (slots <= 8) AH_STRIP(8);
     else if (slots <= 16) AH_STRIP(16);

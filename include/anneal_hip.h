@@ -292,7 +292,8 @@ int ah_softmax_ce(ah_device *dev, const float *z, const int32_t *labels, int32_t
                   float *loss);
 
 /* Config-5 chain: Y = Shrink(Pad(Permute(X,(1,0)))), S = softmax(Y, 1),
- * out = S * recip(sqrt(mean(S*S,1) + 1e-6)) * g; loss = Sum(out); returns dX [R,Cc], dg [Cc]. */
+ * out = S * recip(sqrt(mean(S*S,1) + 1e-6)) * g; loss = Sum(out); returns dX [R,Cc], dg [Cc]. dX may be X and
+ * dg may be g. */
 int ah_chain_step(ah_device *dev, const float *X, const float *g, int32_t R, int32_t Cc, float *dX, float *dg,
                   float *loss);
 /* ah_chain_step without allocation. No counterpart in the reference: it is for callers that cannot

@@ -4,6 +4,8 @@ Tolerances: f32 contractions and reductions 1e-4 norm-wise
 (max|a-b| / max|b|); f16 outputs within one f16 ulp of the f64-accumulated value rounded at the same
 points; index/tie work bit-exact.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -282,6 +284,41 @@ def test_chain_infinite_entries(dev, R, Cc, spin):
         assert np.isnan(got[:, bad]).all() and np.isnan(out[11][bad]).all() and np.isnan(out[12][0])
     else:
         assert np.allclose(out[12][0], (g * dg).sum(), rtol=1e-5)
+
+
+@pytest.mark.parametrize("R,Cc", [(1, 4), (64, 36), (1025, 100), (4096, 260), (4097, 64), (8192, 96), (9000, 8)])
+@pytest.mark.parametrize("same", ["X", "g", "both"])
+def test_chain_in_place(dev, R, Cc, same):
+    """dX written over X, dg over g: through both entry points, and through the item's kernel with spin = 0, where a workgroup
+    whose strip's other parts have not arrived takes their statistics from X at once. Against the float64 closed form, with
+    the bound of test_chain_strip_edges."""
+    rng = np.random.default_rng(R + 7 * Cc)
+    X, g = rng.standard_normal((R, Cc)).astype(np.float32), (1 + 0.02 * rng.standard_normal(Cc)).astype(np.float32)
+    x = X.astype(np.float64)
+    m = x.max(0)
+    S = np.exp(x - m) / np.exp(x - m).sum(0)
+    T = np.sqrt((S * S).mean(0) + 1e-6)
+    gS = g / T - S * (g * S.sum(0) / (R * T**3))
+    dX = S * (gS - (gS * S).sum(0))
+    k = C.c_void_p()
+    L.check(dev.lib.ah_module_get(dev.h, f"tmpl:chain;R={R};Cc={Cc};spin=0".encode(), b"kernel", C.byref(k)))
+    one = (C.c_uint32 * 3)(1, 1, 1)
+
+    def item(bX, bg, R, Cc, bdX, bdg, bl):
+        p = (C.c_void_p * 5)(bdX.ptr, bX.ptr, bg.ptr, bdg.ptr, bl.ptr)
+        L.check(dev.lib.ah_launch(dev.h, k, one, one, p, 5, None, 0))
+
+    for call in (dev.chain_step, dev.chain_step_noalloc, item):
+        bX, bg, bl = dev.buffer(X), dev.buffer(g), dev.buffer(1)
+        bdX = bX if same != "g" else dev.buffer(R * Cc)
+        bdg = bg if same != "X" else dev.buffer(Cc)
+        call(bX, bg, R, Cc, bdX, bdg, bl)
+        dev.sync()
+        got = bdX.read().reshape(R, Cc)
+        assert np.all(np.abs(got - dX) <= 16 * 2.0**-23 * (S * g / T) + 4 * 2.0**-24 * (g / T) * (x == m) + 1e-30)
+        assert np.allclose(bdg.read(), 1 / T, rtol=1e-5) and np.allclose(bl.read()[0], (g / T).sum(), rtol=1e-5)
+        for b in {id(b): b for b in (bX, bg, bl, bdX, bdg)}.values():
+            b.free()
 
 
 F16_VARIANTS = list(range(1, 40))   # every gemm16 variant (gemm16_kernel.h Var<V>; 32-39 use 16x16x32 MFMAs)
