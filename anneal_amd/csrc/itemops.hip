@@ -76,47 +76,49 @@ __global__ __launch_bounds__(256) void reduce_rows_kernel(const T *G, int M, int
     if (lane == 0) out[row] = op == RED_MAX ? acc : acc * scale;
 }
 
-// Column reduce. A row group of kColLanes lanes reads V consecutive columns per lane (16 bytes of G), so a block covers
-// kColLanes * V columns and 1024 / kColLanes = 64 rows at a time, four of each thread's rows in flight; the row groups are
-// then folded through LDS in row order (a fixed tree, so the result does not depend on timing). Bound by the read of G:
-// one column per lane and one row in flight took 7.8 us for 4096 x 1024 f16 (8 MiB), and the second pass, one thread per
-// column walking its chunks, 16.7 us; now 4.9 and 4.6 us (cold operands). With Z, an element enters as Where(Z == max(Z, 0), G, 0) (the
-// ReLU backward mask, gradient_ruleset.go:153-161), else 0.
+// Column reduce. A row group of LANES lanes reads V consecutive columns per lane (16 bytes of G), so a block covers LANES * V
+// columns and THREADS / LANES rows at a time, four of each thread's rows in flight; the row groups are then folded through
+// LDS in row order (a fixed tree, so the result does not depend on timing). Bound by the read of G: one column per lane and
+// one row in flight took 7.8 us for 4096 x 1024 f16 (8 MiB), and the second pass, one thread per column walking its chunks,
+// 16.7 us; now 4.9 and 4.6 us (cold operands). With Z, an element enters as Where(Z == max(Z, 0), G, 0) (the ReLU backward
+// mask, gradient_ruleset.go:153-161), else 0.
 // Blocks take `rows` rows each. One chunk (gridDim.y = 1) writes out itself; more leave part[chunk][n] for the fold.
-constexpr int kColLanes = 16, kColThreads = 1024, kColGroups = kColThreads / kColLanes;
+// The operation is a template argument: chosen at run time it was most of the vector work of a single block (512 x 8 f16
+// 10.7 us, so 4.7; 4096 x 1024 f16 7.2, so 6.3 in both launches).
 template <typename T, int V>
-struct ColVec { typedef T type __attribute__((ext_vector_type(V))); };
+struct ColVec { typedef T type __attribute__((ext_vector_type(V), aligned(V * sizeof(T) < 16 ? V * sizeof(T) : 16))); };
 
-template <typename T, typename TZ, int V>
-__global__ __launch_bounds__(kColThreads) void reduce_cols_kernel(const T *G, const TZ *Z, int M, int N, int rows, int op,
-                                                                   float scale, float *part, float *out) {
+template <typename T, typename TZ, int V, int THREADS, int LANES, int OP>
+__global__ __launch_bounds__(THREADS) void reduce_cols_kernel(const T *G, const TZ *Z, int M, int N, int rows, float scale,
+                                                              float *part, float *out) {
+    constexpr int GROUPS = THREADS / LANES, CB = LANES * V, PARTS = GROUPS < 8 ? GROUPS : 8;
     typedef typename ColVec<T, V>::type vt;
     typedef typename ColVec<TZ, V>::type vz;
-    __shared__ float red[kColGroups][kColLanes * V + 1];
-    const int l = threadIdx.x % kColLanes, grp = threadIdx.x / kColLanes;
-    const int c0 = blockIdx.x * (kColLanes * V) + l * V;
+    __shared__ float red[GROUPS][CB + 1];
+    const int l = threadIdx.x % LANES, grp = threadIdx.x / LANES;
+    const int c0 = blockIdx.x * CB + l * V;
     const int r0 = blockIdx.y * rows, r1 = min(M, r0 + rows);
     float acc[V];
 #pragma unroll
-    for (int u = 0; u < V; u++) acc[u] = red_init(op);
+    for (int u = 0; u < V; u++) acc[u] = red_init(OP);
     if (c0 < N) {   // N % V == 0 (or V == 1): a lane's columns are all in or all out
-        for (int r = r0 + grp; r < r1; r += 4 * kColGroups) {
+        for (int r = r0 + grp; r < r1; r += 4 * GROUPS) {
             vt g[4];
             vz z[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const long i = (long)min(r + j * kColGroups, r1 - 1) * N + c0;
+                const long i = (long)min(r + j * GROUPS, r1 - 1) * N + c0;
                 g[j] = *(const vt *)(G + i);
                 if (Z) z[j] = *(const vz *)(Z + i);
             }
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                if (r + j * kColGroups >= r1) break;
+                if (r + j * GROUPS >= r1) break;
 #pragma unroll
                 for (int u = 0; u < V; u++) {
                     float v = (float)g[j][u];
                     if (Z) v = (float)z[j][u] >= 0.0f ? v : 0.0f;
-                    acc[u] = red_step(op, acc[u], v);
+                    acc[u] = red_step(OP, acc[u], v);
                 }
             }
         }
@@ -124,24 +126,24 @@ __global__ __launch_bounds__(kColThreads) void reduce_cols_kernel(const T *G, co
 #pragma unroll
     for (int u = 0; u < V; u++) red[grp][l * V + u] = acc[u];
     __syncthreads();
-    // fold: thread (column, eighth of the row groups), then the eighths in order
-    constexpr int CB = kColLanes * V, PARTS = 8;
+    // fold: thread (column, a PARTS-th of the row groups), then those in order
     __shared__ float red2[PARTS][CB];
-    for (int t = threadIdx.x; t < CB * PARTS; t += kColThreads) {
+    for (int t = threadIdx.x; t < CB * PARTS; t += THREADS) {
         const int c = t % CB, p = t / CB;
-        float v = red[p * (kColGroups / PARTS)][c];
+        float v = red[p * (GROUPS / PARTS)][c];
 #pragma unroll
-        for (int k = 1; k < kColGroups / PARTS; k++) v = red_join(op, v, red[p * (kColGroups / PARTS) + k][c]);
+        for (int k = 1; k < GROUPS / PARTS; k++) v = red_join(OP, v, red[p * (GROUPS / PARTS) + k][c]);
         red2[p][c] = v;
     }
     __syncthreads();
-    const int col = blockIdx.x * CB + threadIdx.x;
-    if ((int)threadIdx.x < CB && col < N) {
-        float v = red2[0][threadIdx.x];
+    for (int t = threadIdx.x; t < CB; t += THREADS) {
+        const int col = blockIdx.x * CB + t;
+        if (col >= N) break;
+        float v = red2[0][t];
 #pragma unroll
-        for (int p = 1; p < PARTS; p++) v = red_join(op, v, red2[p][threadIdx.x]);
+        for (int p = 1; p < PARTS; p++) v = red_join(OP, v, red2[p][t]);
         if (gridDim.y > 1) part[(long)blockIdx.y * N + col] = v;
-        else out[col] = op == RED_MAX ? v : v * scale;
+        else out[col] = OP == RED_MAX ? v : v * scale;
     }
 }
 
@@ -354,23 +356,39 @@ hipError_t reduce_rows(const void *G, bool f16, int M, int N, int op, float scal
     return hipGetLastError();
 }
 
-template <typename T, typename TZ, int V>
-static hipError_t launch_reduce_cols(const void *G, const void *Z, int M, int N, int op, float scale, float *work,
-                                     float *out, hipStream_t s) {
-    // Chunks of 256 rows (4 per thread), doubled in number while the blocks stay within two per CU and a chunk keeps the
-    // kRedRows rows the workspace is sized for: few columns leave the chip to the rows. Up to 512 rows of few enough
-    // blocks go as one chunk: the second launch costs more than the longer walk (256 x 512 f32: 6.0 us as two launches
-    // of 64-row chunks, 4.2 us as one).
-    const int groups = (N + kColLanes * V - 1) / (kColLanes * V);
-    int rows = 4 * kColGroups;
+template <typename T, typename TZ, int V, int THREADS, int LANES>
+static hipError_t launch_reduce_cols_t(const void *G, const void *Z, int M, int N, int op, float scale, float *work,
+                                       float *out, hipStream_t s) {
+    // Chunks of 256 rows, doubled in number while the blocks stay within two per CU and a chunk keeps the kRedRows rows the
+    // workspace is sized for: few columns leave the chip to the rows. Up to 512 rows go as one chunk: the second launch
+    // costs more than the longer walk (256 x 512 f32: 6.0 us as two launches of 64-row chunks, 4.2 us as one).
+    const int groups = (N + LANES * V - 1) / (LANES * V);
+    int rows = 256;
     if (M <= 512) rows = M;
     else while (rows > kRedRows && (long)groups * ((M + rows - 1) / rows) < 512) rows /= 2;
     const int chunks = (M + rows - 1) / rows;
-    hipLaunchKernelGGL((reduce_cols_kernel<T, TZ, V>), dim3(groups, chunks), dim3(kColThreads), 0, s, (const T *)G,
-                       (const TZ *)Z, M, N, rows, op, scale, work, out);
+#define AH_RC(o) hipLaunchKernelGGL((reduce_cols_kernel<T, TZ, V, THREADS, LANES, o>), dim3(groups, chunks), dim3(THREADS), 0, s, \
+                                    (const T *)G, (const TZ *)Z, M, N, rows, scale, work, out)
+    if (op == RED_MAX) AH_RC(RED_MAX);
+    else if (op == RED_SUMSQ) AH_RC(RED_SUMSQ);
+    else AH_RC(RED_SUM);
+#undef AH_RC
     if (chunks > 1)
         hipLaunchKernelGGL(reduce_cols_final_kernel, dim3((N + 31) / 32), dim3(256), 0, s, work, chunks, N, op, scale, out);
     return hipGetLastError();
+}
+
+template <typename T, typename TZ, int V>
+static hipError_t launch_reduce_cols(const void *G, const void *Z, int M, int N, int op, float scale, float *work,
+                                     float *out, hipStream_t s) {
+    // 64 row groups of 16 lanes, except where more than 4096 lanes' worth of columns fill the chip by themselves: few rows
+    // leave most row groups idle (4 x 4000000 f32 165 us, so 17 in blocks of 4 row groups; 8 x 244376 11.6, so 3.8), and
+    // single columns a lane are then read 64 lanes abreast, 256 bytes of f32 (100 x 1000001 f32 233 us, so 83). With fewer
+    // columns and 257 to 512 rows the 64 row groups are 1.6 to 4 times faster than either.
+    const long lanes = ((long)N + V - 1) / V;
+    if (lanes > 4096 && M <= (V == 1 ? 128 : 16)) return launch_reduce_cols_t<T, TZ, V, 256, 64>(G, Z, M, N, op, scale, work, out, s);
+    if (lanes > 4096 && V == 1) return launch_reduce_cols_t<T, TZ, V, 1024, 64>(G, Z, M, N, op, scale, work, out, s);
+    return launch_reduce_cols_t<T, TZ, V, 1024, 16>(G, Z, M, N, op, scale, work, out, s);
 }
 
 template <typename T, typename TZ>

@@ -9,6 +9,8 @@ replayed as HIP graphs (tensor.JIT), on the GPU.
   (backend/webgpu/executor.go:26-237, schedule/exec.go:6-32), and plans replayed as graphs vs eager runs.
 - Run contract: buffers start at zero (a missing or short leaf input leaves zeros).
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -361,3 +363,32 @@ def test_column_reduce_edges(dev, M, N, f16):
                   [Buffer(10, N, [N]), Buffer(1, M * N, [M, N], dt), Buffer(2, M * N, [M, N], dt)])
     got, t = ex.run([it], {1: G.ravel(), 2: Z.ravel()})[10], np.where(Z >= 0, g64, 0.0)
     assert np.all(np.abs(got - t.sum(0)) <= 24 * 2.0**-24 * np.abs(t).sum(0))
+
+
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("M,N", [(1, 4097), (16, 32776), (17, 32776), (64, 4099), (65, 4099), (300, 8200), (515, 4101)])
+def test_column_reduce_wide_edges(dev, M, N, f16):
+    """More than 4096 lanes' worth of columns: the blocks for few rows, and those that read single columns 64 lanes abreast.
+    Sums and maxima, with the bound of test_column_reduce_edges."""
+    test_column_reduce_edges(dev, M, N, f16)
+
+
+def test_column_reduce_wide_rate(dev):
+    """Columns that 16-byte loads do not divide, and few rows of many columns, are read at a rate like that of the aligned
+    shape (2.4 times as long when every block had 16 lanes' columns and 64 row groups)."""
+    def us(M, N):
+        bufs = [dev.buffer(N), dev.buffer(M * N)]
+        k, one = C.c_void_p(), (C.c_uint32 * 3)(1, 1, 1)
+        L.check(dev.lib.ah_module_get(dev.h, f"tmpl:reduce;dtype=f32;op=sum;axis=0;M={M};N={N}".encode(), b"kernel", C.byref(k)))
+        p = (C.c_void_p * 2)(bufs[0].ptr, bufs[1].ptr)
+        best = 1e9
+        for _ in range(6):
+            dev.timer_start()
+            for _ in range(10):
+                L.check(dev.lib.ah_launch(dev.h, k, one, one, p, 2, None, 0))
+            best = min(best, dev.timer_stop() * 100)
+        for b in bufs:
+            b.free()
+        return best
+    few, odd = us(4, 4000000) / us(64, 250000), us(100, 1000001) / us(100, 1000000)
+    assert few < 1.5 and odd < 1.7, (few, odd)
