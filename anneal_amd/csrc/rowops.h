@@ -25,7 +25,7 @@ hipError_t softmax_ce_cols(const float *z, const int32_t *labels, int B, int C, 
                            float *part, hipStream_t s);
 // rowloss (each row's log-probability of its label) and loss (a * their sum) are both optional; loss takes ws,
 // kSoftmaxWsFloats floats, zero before the first call; its counters are left zero.
-constexpr int kSoftmaxWsFloats = 2048;
+constexpr int kSoftmaxWsFloats = 4096;
 hipError_t softmax_ce(const float *z, const int32_t *labels, int B, int C, float a, float *dz, float *rowloss,
                       hipStream_t s, float *loss = nullptr, float *ws = nullptr);
 hipError_t mse_finalize(const float *acc, float scale, float *out, hipStream_t s);

@@ -238,7 +238,9 @@ __global__ __launch_bounds__(kSmWideThreads) void softmax_ce_wide_kernel(const f
     softmax_loss_fold(total, a, loss, ws, red[0]);
 }
 
-// Longer rows: a wave a row, from memory.
+// Longer rows: a wave a row, from memory; with the loss up to kSmLongBlocks workgroups, which fill the chip 8 to a CU (512 of
+// them left it a quarter full: 4096 x 16384 749 us a call, so 513).
+constexpr int kSmLongBlocks = 2048;
 __global__ __launch_bounds__(256) void softmax_ce_long_kernel(const float *z, const int32_t *labels, int B, int C,
                                                               float a, float *dz, float *rowloss, float *loss, float *ws) {
     __shared__ float red[4];
@@ -1164,7 +1166,7 @@ hipError_t softmax_ce(const float *z, const int32_t *labels, int B, int C, float
                       hipStream_t s, float *loss, float *ws) {
     if (B <= 0) return hipSuccess;
     if (loss && !ws) return hipErrorInvalidValue;
-    static_assert(kSoftmaxWsFloats >= kSmSlots + 2 * kSmBlocks, "one slot a workgroup");
+    static_assert(kSoftmaxWsFloats >= kSmSlots + 2 * kSmBlocks && kSoftmaxWsFloats >= kSmSlots + kSmLongBlocks, "one slot a workgroup");
     if (C <= 1024) {
         const int waves = std::min(kSmWaves, (B + kSmBlocks - 1) / kSmBlocks);
         const dim3 grid(std::min(kSmBlocks, (B + waves - 1) / waves)), block(64 * waves);
@@ -1183,7 +1185,7 @@ hipError_t softmax_ce(const float *z, const int32_t *labels, int B, int C, float
         else AH_SM(16);
 #undef AH_SM
     } else {
-        hipLaunchKernelGGL(softmax_ce_long_kernel, dim3(loss ? std::min(2 * kSmBlocks, (B + 3) / 4) : (B + 3) / 4), dim3(256), 0, s, z,
+        hipLaunchKernelGGL(softmax_ce_long_kernel, dim3(loss ? std::min(kSmLongBlocks, (B + 3) / 4) : (B + 3) / 4), dim3(256), 0, s, z,
                            labels, B, C, a, dz, rowloss, loss, ws);
     }
     return hipGetLastError();

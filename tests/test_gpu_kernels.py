@@ -173,6 +173,36 @@ def test_softmax_ce_edges(dev, B, C):
     assert np.abs(out[13] - rows).max() <= 1e-5 * max(1.0, np.abs(rows).max())
 
 
+def test_softmax_ce_long_rows(dev):
+    """Rows of more than 8192 logits, more of them than workgroups times waves (each wave then takes several): against the
+    item, which computes the same rows one to a wave and no loss (the same bits, and the loss within 1e-5 of the rows' sum);
+    and the call takes no longer than the item's kernel by more than a quarter (twice as long with 512 workgroups)."""
+    B, C_ = 8200, 8200
+    z, lab = RNG.standard_normal((B, C_), dtype=np.float32), RNG.integers(0, C_, B).astype(np.int32)
+    bz, bl, bd, bs = dev.buffer(z), dev.buffer(lab, L.AH_I32), dev.buffer(B * C_), dev.buffer(1)
+    bd2, br = dev.buffer(B * C_), dev.buffer(B)
+    k, one = C.c_void_p(), (C.c_uint32 * 3)(1, 1, 1)
+    L.check(dev.lib.ah_module_get(dev.h, f"tmpl:softmax_ce;B={B};C={C_}".encode(), b"kernel", C.byref(k)))
+    p = (C.c_void_p * 4)(bd2.ptr, bz.ptr, bl.ptr, br.ptr)
+
+    def ms(call):
+        best = 1e9
+        for _ in range(5):
+            dev.timer_start()
+            call()
+            best = min(best, dev.timer_stop())
+        return best
+
+    item = ms(lambda: L.check(dev.lib.ah_launch(dev.h, k, one, one, p, 4, None, 0)))
+    call = ms(lambda: dev.softmax_ce(bz, bl, B, C_, bd, bs))
+    assert np.array_equal(bd.read().view(np.uint32), bd2.read().view(np.uint32))
+    want = -br.read().astype(np.float64).sum() / B
+    assert abs(bs.read()[0] - want) <= 1e-5 * abs(want)
+    for b in (bz, bl, bd, bs, bd2, br):
+        b.free()
+    assert call < 1.25 * item, (call, item)
+
+
 # (4096, 256), (8192, 64) and (8192, 528): the column-strip kernel that holds X on chip; the others: the
 # three-kernel chain
 @pytest.mark.parametrize("R,Cc,grow", [(64, 32, False), (257, 260, False), (1024, 512, False), (4096, 256, False),
