@@ -495,6 +495,18 @@ static bool use_dot(const GemmDesc &d) {
     return d.ta == 0 && d.tb == 0 && d.tile == 0 && (long)d.M * d.N <= 16384 && d.K >= 256;
 }
 
+// f16 contractions the dot kernel takes although the MFMA kernels admit them: those that ask for no particular kernel and no
+// partial sums. Its time grows with the products (every output reads its row of A and of B), the split kernel's (gemm16s.hip)
+// with K alone: 3 x 1000 x 2048 4.8 us against 7.7, 64 x 64 x 8200 8.7 against 11.1; they meet at about 2^25 products (16 x
+// 512 x 4104 7.5 against 9.8, 4 x 1000 x 8200 12.6 against 11.4, 16 x 512 x 8200 13.6 against 11.6), and at half of that with
+// more than 8192 outputs of 8 rows and more (8 x 2048 x 1032 6.4 against 7.7, 8 x 1752 x 1832 9.9 against 7.9). One or two
+// rows take it at any K (1 x 4096 x 4096 7.2 against 10.6).
+static bool dot16(const GemmDesc &d) {
+    if (d.variant || d.splits || d.kgroups || d.colsum || d.epi == EPI_MSE || d.A2 || d.C2 || !use_dot(d)) return false;
+    const long outs = (long)d.M * d.N;
+    return d.M <= 2 || outs * d.K <= 1L << (outs > 8192 && d.M >= 8 && d.N >= 8 ? 24 : 25);
+}
+
 template <typename T>
 static hipError_t launch_layout(const GemmDesc &d, hipStream_t s) {
     if (use_dot(d)) return launch_dot<T>(d, s);
@@ -512,6 +524,7 @@ hipError_t gemm_launch(const GemmDesc &d, hipStream_t s) {
     if (d.K < 0) return hipErrorInvalidValue;
     if (d.dtype == GEMM_F16) {
         hipError_t e = hipSuccess;
+        if (dot16(d)) return launch_dot<half_t>(d, s);
         if (gemm16s_try_launch(d, s, &e)) return e;
         if (gemm16_try_launch(d, s, &e)) return e;
         if (d.A2) return hipErrorInvalidValue;   // two-plane contractions run on the direct-to-LDS kernels only

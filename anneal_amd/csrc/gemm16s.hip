@@ -80,13 +80,11 @@ static bool choose(const GemmDesc &d, G16SPlan *best) {
 // against 19.9 / 23.2 / 24.0 here (NT / N,MN / MN,MN), 2048 x 2048 x 2048 24.5 / 25.2 / 30.9 against 27.4 / 32.3 / 32.0,
 // 4096 x 4096 x 2048 62 / 68 / 105 against 75 / 88 / 104. (Between 64 and 96 tiles this kernel is
 // the faster one, 1024 x 1024 x 2048 16.0 / 17.3 / 17.7 us against 21.2 / 21.3 / 23.2, but adds K in another order than the
-// variants the BEAM search may substitute for an unedited key, which it takes only bit for bit.) One or two rows of a product with
-// few outputs stay with the dot kernel (1 x 4096 x 4096 7.2 us against 10.6).
+// variants the BEAM search may substitute for an unedited key, which it takes only bit for bit.)
 bool gemm16s_try_launch(const GemmDesc &d, hipStream_t s, hipError_t *err) {
     if (d.dtype != GEMM_F16 || d.K <= 0 || d.epi == EPI_MSE || d.colsum || d.A2 || d.C2 || (d.ta && !d.tb)) return false;
     if (d.tile || d.variant || d.splits || d.kgroups) return false;   // the caller's choice of kernel
     if (!operand_ok(d.A, d.lda, d.ta, d.M, d.K) || !operand_ok(d.B, d.ldb, d.tb, d.N, d.K)) return false;
-    if (!d.ta && !d.tb && d.M <= 2 && (long)d.M * d.N <= 16384 && d.K >= 256) return false;
     const long t256 = (long)((d.M + 255) / 256) * ((d.N + 255) / 256), t128 = (long)((d.M + 127) / 128) * ((d.N + 127) / 128);
     const int tile = t256 >= 224 ? 256 : 128;
     const uintptr_t al = (uintptr_t)d.C | (uintptr_t)d.aux | (uintptr_t)d.bias | (uintptr_t)d.W32 | (uintptr_t)d.W16 | (uintptr_t)d.gout;

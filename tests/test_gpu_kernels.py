@@ -756,3 +756,26 @@ def test_gemm16_split_kernel_unaligned_output(dev):
     assert np.all(np.abs(C[:, :N] - ref) <= 2.0**-11 * np.abs(ref) + 1e-3) and np.all(C[:, N:] == 7)
     for b in (dA, dB, dC):
         b.free()
+
+
+def gemm16_bits(dev, M, N, K, ta=0, tb=0, variant=0, rows=None):
+    """The f32 bits of the sums (an SGD step of 1 from zero weights) on fixed operands, or of the first `rows` rows of A."""
+    rng = np.random.default_rng(M * 31 + N * 7 + K)
+    As, Bs = store_operand(q16(rng.standard_normal((M, K))), ta), store_operand(q16(rng.standard_normal((N, K))), tb)
+    dA, dB, dW = dev.buffer(As.astype(np.float16), L.AH_F16), dev.buffer(Bs.astype(np.float16), L.AH_F16), dev.buffer(np.zeros(M * N, np.float32))
+    m = rows or M
+    dev.gemm(dtype=L.AH_F16, epi=L.EPI_SGD, ta=ta, tb=tb, M=m, N=N, K=K, A=dA, B=dB, lda=As.shape[1], ldb=Bs.shape[1], ldc=N,
+             scale=1.0, W32=dW, lr=-1.0, variant=variant)
+    out = dW.read().view(np.uint32).reshape(M, N)[:m].copy()
+    for b in (dA, dB, dW):
+        b.free()
+    return out
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 1000, 2048), (8, 320, 6544), (8, 64, 4096), (27, 64, 296), (16, 512, 4096), (64, 64, 8192)])
+def test_gemm16_few_outputs_take_the_dot_kernel(dev, M, N, K):
+    """Up to 2^25 products of at most 16384 outputs: a wave an output, as for one row (the split kernel took twice the time),
+    and so the bits of one row alone."""
+    C = gemm16_bits(dev, M, N, K)
+    np.testing.assert_array_equal(C[:1], gemm16_bits(dev, M, N, K, rows=1))
+    np.testing.assert_array_equal(C[:2], gemm16_bits(dev, M, N, K, rows=2))
