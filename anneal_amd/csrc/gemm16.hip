@@ -74,11 +74,15 @@ bool gemm16_variant_params(int v, G16Params *out) {
 //    K must split into two groups of whole stages; otherwise 14 (four stages in flight): 40.9 / 41.8 / 47.0.
 //  - more 128x128 tiles than CUs: 1, whose 64 KiB of LDS let two tiles share a CU (35 and 14 hold 128 KiB): 2048 x 4096
 //    x 1024 24.0 / 27.8 / 39.8 us against 27.5 / 30.0 / 41.9.
+//  - short K, where filling and draining more stages or k-groups, or a 16x16x32 tile's epilogue, costs more than they give:
+//    3 again up to K = 128 (8192 x 8192 x 64 NT 47.4 us against 54.1 with 39, 4096 x 4096 x 128 14.4 against 15.7; x 256 19.8
+//    against 19.4), 1 again below K = 256 (2048 x 2048 x 128 6.7 / 8.8 us against 8.2 / 9.7 with 35, 2048 x 1024 x 192 7.0
+//    against 7.6 with 14) and for both operands along K up to 512 (512 x 6272 x 512 11.4 against 12.2, x 576 on even).
 int gemm16_default_variant(const GemmDesc &d) {
     const long t256 = (long)((d.M + 255) / 256) * ((d.N + 255) / 256);
     const long t128 = (long)((d.M + 127) / 128) * ((d.N + 127) / 128);
-    if (d.tile == 256 || (d.tile == 0 && t256 >= 224)) return 39;
-    if (t128 > 256) return 1;
+    if (d.tile == 256 || (d.tile == 0 && t256 >= 224)) return d.K <= 128 ? 3 : 39;
+    if (t128 > 256 || d.K < 256 || (!d.ta && !d.tb && d.K <= 512)) return 1;
     return d.K % 128 == 0 ? 35 : 14;
 }
 

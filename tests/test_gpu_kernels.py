@@ -779,3 +779,11 @@ def test_gemm16_few_outputs_take_the_dot_kernel(dev, M, N, K):
     C = gemm16_bits(dev, M, N, K)
     np.testing.assert_array_equal(C[:1], gemm16_bits(dev, M, N, K, rows=1))
     np.testing.assert_array_equal(C[:2], gemm16_bits(dev, M, N, K, rows=2))
+
+
+@pytest.mark.parametrize("shape", [(0, 0, 1024, 1024, 128), (0, 1, 1024, 1024, 128), (1, 1, 1024, 1152, 128), (0, 0, 1024, 1024, 512)],
+                         ids=lambda s: "ta%d_tb%d_%dx%dx%d" % s)
+def test_gemm16_short_k_keeps_one_k_group(dev, shape):
+    """Whole tiles and a short K: variant 1's sums (one run over K), not those of two k-groups."""
+    ta, tb, M, N, K = shape
+    np.testing.assert_array_equal(gemm16_bits(dev, M, N, K, ta, tb), gemm16_bits(dev, M, N, K, ta, tb, variant=1))
