@@ -81,6 +81,16 @@ static bool choose(const GemmDesc &d, G16SPlan *best) {
 // 4096 x 4096 x 2048 62 / 68 / 105 against 75 / 88 / 104. (Between 64 and 96 tiles this kernel is
 // the faster one, 1024 x 1024 x 2048 16.0 / 17.3 / 17.7 us against 21.2 / 21.3 / 23.2, but adds K in another order than the
 // variants the BEAM search may substitute for an unedited key, which it takes only bit for bit.)
+// They also keep ragged outputs of both operands along K (NT) whose epilogue reads no matrix: only the edge tiles then store
+// element by element. 3584 x 7040 x 128 22.8 us there against 31.1 here, 6709 x 6656 x 320 58.8 against 71.7, 905 x 5120 x 1088
+// 21.9 against 27.4, over 256 tiles on average 1.13 times faster (0.89 to 1.36, 80 shapes); over 192 tiles up to K = 1280
+// (923 x 3840 x 128 7.2 against 9.0), over 128 with K from 384 (3477 x 768 x 640 12.7 against 14.8); with fewer tiles, or a
+// longer K, K split here gains. In the other layouts or with a mask or SGD epilogue this kernel takes half the time.
+static bool whole_tiles(const GemmDesc &d, long t128) {
+    if (d.K % 64 || d.ta || d.tb || d.epi == EPI_MASK || d.epi == EPI_SGD) return false;
+    return t128 > 256 || (d.K <= 1280 && (t128 > 192 || (t128 > 128 && d.K >= 384)));
+}
+
 bool gemm16s_try_launch(const GemmDesc &d, hipStream_t s, hipError_t *err) {
     if (d.dtype != GEMM_F16 || d.K <= 0 || d.epi == EPI_MSE || d.colsum || d.A2 || d.C2 || (d.ta && !d.tb)) return false;
     if (d.tile || d.variant || d.splits || d.kgroups) return false;   // the caller's choice of kernel
@@ -88,8 +98,9 @@ bool gemm16s_try_launch(const GemmDesc &d, hipStream_t s, hipError_t *err) {
     const long t256 = (long)((d.M + 255) / 256) * ((d.N + 255) / 256), t128 = (long)((d.M + 127) / 128) * ((d.N + 127) / 128);
     const int tile = t256 >= 224 ? 256 : 128;
     const uintptr_t al = (uintptr_t)d.C | (uintptr_t)d.aux | (uintptr_t)d.bias | (uintptr_t)d.W32 | (uintptr_t)d.W16 | (uintptr_t)d.gout;
-    if (t128 >= 64 && d.M % tile == 0 && d.N % tile == 0 && d.K % 64 == 0 && d.ldc % 4 == 0 && d.ldaux % 4 == 0 && (al & 15) == 0)
-        return false;
+    const bool aligned = d.ldc % 4 == 0 && d.ldaux % 4 == 0 && (al & 15) == 0;
+    if (aligned && t128 >= 64 && d.M % tile == 0 && d.N % tile == 0 && d.K % 64 == 0) return false;
+    if (aligned && whole_tiles(d, t128)) return false;
     G16SPlan p;
     if (!choose(d, &p)) return false;
     *err = launch_cfg(d, p, s);

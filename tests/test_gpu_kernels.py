@@ -758,12 +758,21 @@ def test_gemm16_split_kernel_unaligned_output(dev):
         b.free()
 
 
-def gemm16_bits(dev, M, N, K, ta=0, tb=0, variant=0, rows=None):
-    """The f32 bits of the sums (an SGD step of 1 from zero weights) on fixed operands, or of the first `rows` rows of A."""
+def gemm16_bits(dev, M, N, K, ta=0, tb=0, variant=0, rows=None, store=False):
+    """The f32 bits of the sums (an SGD step of 1 from zero weights) on fixed operands, or of the first `rows` rows of A; with
+    store, the f16 bits of a scaled store instead."""
     rng = np.random.default_rng(M * 31 + N * 7 + K)
     As, Bs = store_operand(q16(rng.standard_normal((M, K))), ta), store_operand(q16(rng.standard_normal((N, K))), tb)
     dA, dB, dW = dev.buffer(As.astype(np.float16), L.AH_F16), dev.buffer(Bs.astype(np.float16), L.AH_F16), dev.buffer(np.zeros(M * N, np.float32))
     m = rows or M
+    if store:
+        dC = dev.buffer(M * N, L.AH_F16)
+        dev.gemm(dtype=L.AH_F16, epi=L.EPI_STORE, ta=ta, tb=tb, M=m, N=N, K=K, A=dA, B=dB, lda=As.shape[1], ldb=Bs.shape[1], ldc=N,
+                 scale=1.0 / 3, C_out=dC, variant=variant)
+        out = dC.read().view(np.uint16).reshape(M, N)[:m].copy()
+        for b in (dA, dB, dW, dC):
+            b.free()
+        return out
     dev.gemm(dtype=L.AH_F16, epi=L.EPI_SGD, ta=ta, tb=tb, M=m, N=N, K=K, A=dA, B=dB, lda=As.shape[1], ldb=Bs.shape[1], ldc=N,
              scale=1.0, W32=dW, lr=-1.0, variant=variant)
     out = dW.read().view(np.uint32).reshape(M, N)[:m].copy()
@@ -787,3 +796,12 @@ def test_gemm16_short_k_keeps_one_k_group(dev, shape):
     """Whole tiles and a short K: variant 1's sums (one run over K), not those of two k-groups."""
     ta, tb, M, N, K = shape
     np.testing.assert_array_equal(gemm16_bits(dev, M, N, K, ta, tb), gemm16_bits(dev, M, N, K, ta, tb, variant=1))
+
+
+@pytest.mark.parametrize("M,N,K,variant", [(2100, 2056, 1024, 1), (1500, 2304, 704, 1), (1031, 3080, 1152, 35), (1100, 2312, 768, 35),
+                                           (4000, 3600, 320, 3)])
+def test_gemm16_ragged_nt_takes_whole_tiles(dev, M, N, K, variant):
+    """Ragged outputs of many tiles, both operands along K: the sums of the whole-tile variant of that size (the split kernel adds
+    the k-steps of its wave sets, which shows where two k-groups are the variant)."""
+    C = gemm16_bits(dev, M, N, K, store=True)
+    np.testing.assert_array_equal(C, gemm16_bits(dev, M, N, K, variant=variant, store=True))
