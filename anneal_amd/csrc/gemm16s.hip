@@ -85,7 +85,9 @@ static bool choose(const GemmDesc &d, G16SPlan *best) {
 // element by element. 3584 x 7040 x 128 22.8 us there against 31.1 here, 6709 x 6656 x 320 58.8 against 71.7, 905 x 5120 x 1088
 // 21.9 against 27.4, over 256 tiles on average 1.13 times faster (0.89 to 1.36, 80 shapes); over 192 tiles up to K = 1280
 // (923 x 3840 x 128 7.2 against 9.0), over 128 with K from 384 (3477 x 768 x 640 12.7 against 14.8); with fewer tiles, or a
-// longer K, K split here gains. In the other layouts or with a mask or SGD epilogue this kernel takes half the time.
+// longer K, K split here gains. A K of less than two stages that 64 does not divide goes to the register-staged kernel's 64x64
+// tiles from 65 to 192 128x128 ones: 256 x 5696 x 32 4.6 us against 5.7, 1044 x 1088 x 56 5.1 against 6.0, 2014 x 1816 x 104 on
+// even (1.12 times faster over 45 shapes; below and above the two are within 3%). In the other layouts or with a mask or SGD epilogue this kernel takes half the time.
 static bool whole_tiles(const GemmDesc &d, long t128) {
     if (d.K % 64 || d.ta || d.tb || d.epi == EPI_MASK || d.epi == EPI_SGD) return false;
     return t128 > 256 || (d.K <= 1280 && (t128 > 192 || (t128 > 128 && d.K >= 384)));
@@ -101,6 +103,7 @@ bool gemm16s_try_launch(const GemmDesc &d, hipStream_t s, hipError_t *err) {
     const bool aligned = d.ldc % 4 == 0 && d.ldaux % 4 == 0 && (al & 15) == 0;
     if (aligned && t128 >= 64 && d.M % tile == 0 && d.N % tile == 0 && d.K % 64 == 0) return false;
     if (aligned && whole_tiles(d, t128)) return false;
+    if (!d.ta && !d.tb && d.epi != EPI_MASK && d.epi != EPI_SGD && d.K < 128 && d.K % 64 && t128 > 64 && t128 <= 192) return false;
     G16SPlan p;
     if (!choose(d, &p)) return false;
     *err = launch_cfg(d, p, s);

@@ -805,3 +805,16 @@ def test_gemm16_ragged_nt_takes_whole_tiles(dev, M, N, K, variant):
     the k-steps of its wave sets, which shows where two k-groups are the variant)."""
     C = gemm16_bits(dev, M, N, K, store=True)
     np.testing.assert_array_equal(C, gemm16_bits(dev, M, N, K, variant=variant, store=True))
+
+
+@pytest.mark.parametrize("M,N,K", [(256, 5696, 32), (1044, 1088, 56), (2100, 1500, 104), (1153, 1024, 8)])
+def test_gemm16_short_ragged_k(dev, M, N, K):
+    """A short K that 64 does not divide, 65 to 192 tiles: the register-staged kernel's bits (which a fixed variant runs here, as
+    no whole-tile variant takes such a K), and float64 within the bound of the split kernel's test."""
+    C = gemm16_bits(dev, M, N, K, store=True)
+    np.testing.assert_array_equal(C, gemm16_bits(dev, M, N, K, variant=1, store=True))
+    rng = np.random.default_rng(M * 31 + N * 7 + K)
+    A, B = q16(rng.standard_normal((M, K))).astype(np.float64), q16(rng.standard_normal((N, K))).astype(np.float64)
+    got = C.view(np.float16).astype(np.float64)
+    acc = (K + 16) * 2.0**-24 * (np.abs(A) @ np.abs(B).T)
+    assert np.all(np.abs(got - (A @ B.T) / 3) <= acc / 3 + 2.0**-11 * np.abs(got) * 1.01 + 2.0**-23)
