@@ -66,7 +66,8 @@ long chain_sync_max_ints();
 // device `ordinal` (the current device at the call).
 long chain_scratch_floats();
 hipError_t chain_scratch_init(int ordinal, float **out);
-// True where the chain runs as one launch, each 32-column strip of X held on chip (one pass over HBM).
+// True where the chain runs as one launch, each 32-column strip of X held on chip (one pass over HBM): where that fits and is
+// the faster.
 bool chain_resident_fits(int R, int Cc);
 // The whole config-5 chain (phase -1: the strip kernel where it fits, else the three kernels below) or one of its three
 // kernels (phase 0 stats, 1 finalize, 2 gradient). work: chain_workspace_floats floats, or chain_array_floats with the

@@ -947,11 +947,17 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
     }
 }
 
-// Parts per strip and rows per part: as few parts as hold the rows on chip, then more while the workgroups stay within one
-// per CU and each keeps 8 slots (512 rows). Two workgroups per CU: 4096 x 4096 34.7 us for 31.8, 3008 x 2048 19.9 for 18.4;
-// parts of 256 rows: 512 x 2048 9.3 us for 8.8, 1024 x 64 8.6 for 9.8. Against the three kernels this is faster at every
-// shape measured from 64 x 64 (6.1 us for 11.3) over 4096 x 64 (10.5 for 14.8), 2048 x 2048 (15.8 for 17.4), 16384 x 64 (13.9
-// for 14.5) and 16384 x 1024 (34.5 for 44.9) to 8192 x 4096, so they are left the shapes that do not fit.
+// Parts per strip and rows per part: the fewest parts of 64 slots that hold the rows (a plan of more than kStripMaxPartsFull
+// parts of more than 45 slots does not fit), then more while the workgroups stay within one per CU and each keeps 8 slots (512
+// rows). Two workgroups per CU: 4096 x 4096 34.7 us for 31.8, 3008 x 2048 19.9 for 18.4; parts of 256 rows: 512 x 2048 9.3 us
+// for 8.8, 1024 x 64 8.6 for 9.8. Against the three kernels this is faster at every shape measured of at most one workgroup
+// per CU, from 64 x 64 (6.1 us for 11.3) over 4096 x 64 (10.5 for 14.8), 2048 x 2048 (15.8 for 17.4), 16384 x 64 (13.9 for
+// 14.5) and 16384 x 1024 (34.5 for 44.9) to 8192 x 4096. Parts of many rows fill their CU, so one more than 256 of them makes
+// a second round, and a round neither loads nor stores all the time: 7000 x 4100 (258 workgroups) 96 us for 74 with X in
+// memory and 74 for 71 with it in the Infinity Cache, 8192 x 5120 111 for 104 and 110 for 86, 7000 x 8192 145 for 128 and 142
+// for 122; strips of one part and up to 48 slots are on even (3000 x 8196 75 for 71 and 59 for 68). The three kernels take
+// those, unless X outgrows the Infinity Cache, which serves their second read of it (16000 x 4096 132 for 148), and X of a few
+// rows on more than two rounds (2 x 27724 19.0 for 15.8).
 struct StripPlan {
     int parts, rows;
 };
@@ -969,7 +975,11 @@ bool chain_resident_fits(int R, int Cc) {
     if (R <= 0 || Cc <= 0 || Cc % 4 || (long)R * Cc * 4 >= (1L << 31)) return false;
     if ((Cc + kStripCols - 1) / kStripCols > kStripMaxStrips) return false;
     const StripPlan p = strip_plan(R, Cc);
-    return p.rows <= kStripRows * (p.parts <= kStripMaxPartsFull ? kStripMaxSlots : kStripMaxRegs);
+    const int strips = (Cc + kStripCols - 1) / kStripCols, slots = p.rows / kStripRows;
+    if (slots > (p.parts <= kStripMaxPartsFull ? kStripMaxSlots : kStripMaxRegs)) return false;
+    if (R < 8 && strips > 512) return false;
+    const bool rounds = strips * p.parts > 256 && slots > (p.parts > 1 ? 32 : 48);
+    return !rounds || (Cc % kStripCols == 0 && (long)R * Cc * 4 > 250000000L);
 }
 
 template <int NS>

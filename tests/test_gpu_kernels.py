@@ -11,6 +11,7 @@ import pytest
 
 import oracle_lib as O
 from anneal_amd import _lib as L
+from anneal_amd.backend import Trainer
 from anneal_amd.executor import Buffer, ExecItem, Executor
 
 pytestmark = pytest.mark.gpu
@@ -203,8 +204,7 @@ def test_softmax_ce_long_rows(dev):
     assert call < 1.25 * item, (call, item)
 
 
-# (4096, 256), (8192, 64) and (8192, 528): the column-strip kernel that holds X on chip; the others: the
-# three-kernel chain
+# The column-strip kernel that holds X on chip, in one part and several (test_chain_three_kernels has the shapes it leaves)
 @pytest.mark.parametrize("R,Cc,grow", [(64, 32, False), (257, 260, False), (1024, 512, False), (4096, 256, False),
                                        (8192, 64, False), (8192, 528, False), (4096, 256, True), (8192, 64, True)])
 def test_chain_kernel_vs_oracle(dev, R, Cc, grow):
@@ -236,7 +236,7 @@ def test_chain_kernel_vs_oracle(dev, R, Cc, grow):
 
 
 # Row counts around the strip kernel's slots (64 rows), parts (4096 rows, or fewer for few columns) and instances; columns
-# that end inside a 32-column strip, one strip, more strips than CUs; beyond its reach (40960 rows: the three-kernel chain)
+# that end inside a 32-column strip, one strip, more strips than CUs; 16 parts of 40 slots
 @pytest.mark.parametrize("R,Cc", [(1, 4), (64, 36), (65, 32), (513, 64), (1025, 100), (2049, 260), (2881, 8200), (3001, 2052),
                                   (4097, 64), (5000, 132), (8192, 96), (9000, 8), (16384, 32), (40960, 4)])
 @pytest.mark.parametrize("spin", [-1, 0])
@@ -274,6 +274,47 @@ def test_chain_strip_edges(dev, R, Cc, spin):
     if spin == 0:
         for k, v in run(-1).items():
             np.testing.assert_array_equal(out[k].view(np.uint32), v.view(np.uint32))
+
+
+@pytest.mark.parametrize("R,Cc,strips", [(8192, 4096, True), (4096, 8192, True), (3000, 8196, True), (16000, 1028, True), (64, 20000, True),
+                                         (5000, 4100, False), (7000, 4100, False), (4096, 8196, False), (9000, 3072, False),
+                                         (2, 27724, False), (16000, 4096, True)])
+def test_chain_route(dev, R, Cc, strips):
+    """The strips take what fits on chip in one round of workgroups; a second round of large ones, and few rows of very many
+    columns, are the three kernels' (test_chain_three_kernels has their results)."""
+    t = Trainer(dev, L.TRAIN_CHAIN, [R, Cc])
+    names = t.kernel_names(R)
+    t.close()
+    assert names == (["chain_resident"] if strips else ["chain_stats", "chain_finalize", "chain_grad"])
+
+
+# More strips than the counters, one more part than a round holds, a few rows, few and many row chunks; columns that end inside
+# a block of 256 and inside a finalize block of 16
+@pytest.mark.parametrize("R,Cc", [(46081, 4), (5000, 4100), (4097, 4364), (2, 27724), (33, 33000), (7, 16420)])
+def test_chain_three_kernels(dev, R, Cc):
+    """Shapes that run chain_stats, chain_finalize and chain_grad, with masked entries (-FLT_MAX and -inf) and ties, against
+    the float64 closed form: the bound of test_chain_strip_edges, twice the terms (the op order rounds the factors of dX an
+    element at a time)."""
+    t = Trainer(dev, L.TRAIN_CHAIN, [R, Cc])
+    assert t.kernel_names(R) == ["chain_stats", "chain_finalize", "chain_grad"]
+    rng = np.random.default_rng(R + Cc)
+    X = rng.standard_normal((R, Cc)).astype(np.float32)
+    X[R // 2, ::3] = X[R - 1, ::3]                           # a tie, maybe of the maximum
+    X[: R // 2, 1], X[: R // 2, 2] = np.float32(-3.4028234663852886e38), -np.inf
+    g = (1 + 0.02 * rng.standard_normal(Cc)).astype(np.float32)
+    t.set("X", X)
+    t.set("g", g)
+    t.step(R)
+    got, dg, loss = t.get("dX", R * Cc).reshape(R, Cc), t.get("dg", Cc), t.get("loss", 1)[0]
+    t.close()
+    x = X.astype(np.float64)
+    m = x.max(0)
+    S = np.exp(x - m) / np.exp(x - m).sum(0)
+    T = np.sqrt((S * S).mean(0) + 1e-6)
+    gS = g / T - S * (g * S.sum(0) / (R * T**3))
+    dX = S * (gS - (gS * S).sum(0))
+    assert np.all(np.abs(got - dX) <= 32 * 2.0**-23 * (S * g / T) + 8 * 2.0**-24 * (g / T) * (x == m) + 1e-30)
+    assert np.allclose(dg, 1 / T, rtol=1e-5) and np.allclose(loss, (g / T).sum(), rtol=1e-5)
 
 
 # One slot (64 rows), a part of 512 rows, several parts, whole strips of one workgroup
