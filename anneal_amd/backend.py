@@ -94,7 +94,8 @@ class Device:
 
     def gemm_tune(self, iterations: int = 3, **kw):
         """Times every f16 variant (or f32 configuration) of the contraction and caches the fastest;
-        returns (variant or configuration index, mean us)."""
+        returns (variant or configuration index, mean us), variant 0 where the kernel that an f16 call runs
+        by itself is no variant and the fastest (nothing is cached then)."""
         d = self._gemm_desc(**kw)
         v, us = C.c_int32(), C.c_double()
         L.check(self.lib.ah_gemm_tune(self.h, C.byref(d), iterations, C.byref(v), C.byref(us)))

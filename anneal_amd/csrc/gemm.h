@@ -97,6 +97,9 @@ bool gemm16_pair_try_launch(const GemmDesc &d0, int nsplit, const GemmDesc *d1, 
                             float *part, long part_floats, hipStream_t s, hipError_t *err);
 
 hipError_t gemm_launch(const GemmDesc &d, hipStream_t s);
+// True where an f16 contraction that leaves the choice open runs a kernel that no variant stands for: the split kernel
+// (gemm16s.h) or the dot kernel.
+bool gemm16_beside_variants(const GemmDesc &d);
 bool gemm16_try_launch(const GemmDesc &d, hipStream_t s, hipError_t *err);
 
 // Template parameters of an f16 variant (table Var<V> in gemm16_kernel.h): tile BM x BN, wave layout

@@ -519,6 +519,8 @@ static hipError_t launch_layout(const GemmDesc &d, hipStream_t s) {
     }
 }
 
+bool gemm16_beside_variants(const GemmDesc &d) { return d.dtype == GEMM_F16 && (dot16(d) || gemm16s_serves(d)); }
+
 hipError_t gemm_launch(const GemmDesc &d, hipStream_t s) {
     if (d.M <= 0 || d.N <= 0) return hipSuccess;
     if (d.K < 0) return hipErrorInvalidValue;

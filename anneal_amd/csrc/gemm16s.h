@@ -8,6 +8,7 @@ namespace ah {
 // of 8 and 16-byte aligned, under 2 GiB; the store, bias, mask and SGD epilogues without partial sums) and the shape is
 // one it serves better than the whole-tile variants (gemm16s.hip has the rule); else returns false.
 bool gemm16s_try_launch(const GemmDesc &d, hipStream_t s, hipError_t *err);
+bool gemm16s_serves(const GemmDesc &d);
 
 // One tile configuration: split workgroups per tile, each contracting `stages` K stages.
 struct G16SPlan {

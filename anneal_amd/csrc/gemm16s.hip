@@ -93,7 +93,7 @@ static bool whole_tiles(const GemmDesc &d, long t128) {
     return t128 > 256 || (d.K <= 1280 && (t128 > 192 || (t128 > 128 && d.K >= 384)));
 }
 
-bool gemm16s_try_launch(const GemmDesc &d, hipStream_t s, hipError_t *err) {
+bool gemm16s_serves(const GemmDesc &d) {
     if (d.dtype != GEMM_F16 || d.K <= 0 || d.epi == EPI_MSE || d.colsum || d.A2 || d.C2 || (d.ta && !d.tb)) return false;
     if (d.tile || d.variant || d.splits || d.kgroups) return false;   // the caller's choice of kernel
     if (!operand_ok(d.A, d.lda, d.ta, d.M, d.K) || !operand_ok(d.B, d.ldb, d.tb, d.N, d.K)) return false;
@@ -104,8 +104,12 @@ bool gemm16s_try_launch(const GemmDesc &d, hipStream_t s, hipError_t *err) {
     if (aligned && t128 >= 64 && d.M % tile == 0 && d.N % tile == 0 && d.K % 64 == 0) return false;
     if (aligned && whole_tiles(d, t128)) return false;
     if (!d.ta && !d.tb && d.epi != EPI_MASK && d.epi != EPI_SGD && d.K < 128 && d.K % 64 && t128 > 64 && t128 <= 192) return false;
+    return true;
+}
+
+bool gemm16s_try_launch(const GemmDesc &d, hipStream_t s, hipError_t *err) {
     G16SPlan p;
-    if (!choose(d, &p)) return false;
+    if (!gemm16s_serves(d) || !choose(d, &p)) return false;
     *err = launch_cfg(d, p, s);
     return true;
 }

@@ -20,6 +20,7 @@
 #include "convnet.h"
 #include "mlpce.h"
 #include "gemm.h"
+#include "gemm16s.h"
 #include "itemops.h"
 #include "rowops.h"
 
@@ -155,9 +156,17 @@ static const std::vector<F32Cfg> &f32_cfgs() {
     return v;
 }
 
+// The device's split-K workspace (used by the f32 tiled kernel and the f16 split kernel for shapes with
+// few tiles and a long K).
+static void use_splitk_ws(ah_device *dev, GemmDesc *g) {
+    if (!dev->splitk_ws) return;
+    g->sk_sync = (int *)dev->splitk_ws;
+    g->sk_part = (float *)((char *)dev->splitk_ws + (size_t)kSplitKMaxTiles * 2 * sizeof(int));
+    g->sk_cap = kSplitKPartFloats;
+}
+
 // Launch with the tuned variant (f16) or configuration (f32) when the caller left the choice open, and
-// with the device's split-K workspace (used by the f32 tiled kernel for shapes with few tiles and a
-// long K).
+// with the split-K workspace.
 static hipError_t gemm_run(ah_device *dev, GemmDesc g, hipStream_t s) {
     if (g.variant == 0 && g.dtype == GEMM_F16) {
         auto it = dev->gemm_variant.find(tune_key(g));
@@ -170,12 +179,7 @@ static hipError_t gemm_run(ah_device *dev, GemmDesc g, hipStream_t s) {
             g.tile = c.tile; g.kgroups = c.kg; g.splits = c.splits;
         }
     }
-    if (dev->splitk_ws) {
-        const size_t sync_bytes = (size_t)kSplitKMaxTiles * 2 * sizeof(int);
-        g.sk_sync = (int *)dev->splitk_ws;
-        g.sk_part = (float *)((char *)dev->splitk_ws + sync_bytes);
-        g.sk_cap = kSplitKPartFloats;
-    }
+    use_splitk_ws(dev, &g);
     return gemm_launch(g, s);
 }
 
@@ -184,18 +188,27 @@ hipError_t ah::gemm_dispatch(ah_device *dev, const GemmDesc &g) { return gemm_ru
 // Times every f16 variant of g (as given: its epilogue runs on whatever outputs g names) and caches
 // the fastest for g's shape. Two passes over the variants, each variant's time the lower of its two
 // means of `iters` launches, so one disturbed measurement does not decide the choice.
+// With automatic, the open choice is timed too (0) where it is no variant: the split or the dot kernel
+// (32 x 4096 x 4096 11.6 us, the fastest variant 31). Where it wins nothing is cached, so launches keep
+// it. (On the split kernel only past K = 256 or where 64 does not divide K: below, a variant's number
+// is what a caller gets for a shape of whole stages, and the two are a microsecond or two apart, 512 x
+// 384 x 256 5.6 us against 7.0.) A training step's own tuning leaves it out, as before.
 static int tune_gemm_f32(ah_device *dev, GemmDesc g, int iters, int *best, double *best_us, bool same_bits);
-static int tune_gemm(ah_device *dev, GemmDesc g, int iters, int *best, double *best_us) {
+static int tune_gemm(ah_device *dev, GemmDesc g, int iters, int *best, double *best_us, bool automatic = false) {
     if (g.dtype == GEMM_F32) return tune_gemm_f32(dev, g, iters, best, best_us, false);
     if (g.dtype != GEMM_F16) return set_error(AH_ERR_UNSUPPORTED, "gemm tuning covers the f16 and f32 kernels");
     if (iters <= 0) return set_error(AH_ERR_INVALID, "gemm tuning: iterations must be > 0");
     hipEvent_t e0, e1;
     AH_HIP(hipEventCreateWithFlags(&e0, hipEventDisableSystemFence));   // timing only
     AH_HIP(hipEventCreateWithFlags(&e1, hipEventDisableSystemFence));
+    g.variant = 0;
+    use_splitk_ws(dev, &g);
+    automatic = automatic && gemm16_beside_variants(g) && (g.K > 256 || g.K % 64 || !gemm16s_serves(g));
+    const int first = automatic ? 0 : 1;
     std::vector<float> t(kGemm16Variants + 1, 0.0f);
     hipError_t err = hipSuccess;
     for (int pass = 0; pass < 2 && err == hipSuccess; pass++) {
-        for (int v = 1; v <= kGemm16Variants && err == hipSuccess; v++) {
+        for (int v = first; v <= kGemm16Variants && err == hipSuccess; v++) {
             g.variant = v;
             err = gemm_launch(g, dev->stream);
             if (err == hipSuccess) err = hipEventRecord(e0, dev->stream);
@@ -210,10 +223,11 @@ static int tune_gemm(ah_device *dev, GemmDesc g, int iters, int *best, double *b
     hipEventDestroy(e0);
     hipEventDestroy(e1);
     if (err != hipSuccess) return fail_hip(err, "gemm tuning");
-    int bv = 1;
-    for (int v = 2; v <= kGemm16Variants; v++)
+    int bv = first;
+    for (int v = first + 1; v <= kGemm16Variants; v++)
         if (t[v] < t[bv]) bv = v;
-    dev->gemm_variant[tune_key(g)] = bv;
+    if (bv) dev->gemm_variant[tune_key(g)] = bv;
+    else dev->gemm_variant.erase(tune_key(g));
     if (best) *best = bv;
     if (best_us) *best_us = t[bv] * 1000.0 / iters;
     return AH_OK;
@@ -229,12 +243,7 @@ static int tune_gemm(ah_device *dev, GemmDesc g, int iters, int *best, double *b
 static int tune_gemm_f32(ah_device *dev, GemmDesc g, int iters, int *best, double *best_us, bool same_bits) {
     if (iters <= 0) return set_error(AH_ERR_INVALID, "gemm tuning: iterations must be > 0");
     const std::vector<F32Cfg> &cfgs = f32_cfgs();
-    if (dev->splitk_ws) {
-        const size_t sync_bytes = (size_t)kSplitKMaxTiles * 2 * sizeof(int);
-        g.sk_sync = (int *)dev->splitk_ws;
-        g.sk_part = (float *)((char *)dev->splitk_ws + sync_bytes);
-        g.sk_cap = kSplitKPartFloats;
-    }
+    use_splitk_ws(dev, &g);
     std::vector<char> admitted(cfgs.size(), 1);
     if (same_bits) {
         // the guard runs on hash-filled copies of g's operands (real operands may still be all zero),
@@ -1283,7 +1292,7 @@ int ah_gemm_tune(ah_device *dev, const ah_gemm_desc *d, int32_t iterations, int3
     g.aux = d->aux; g.ldaux = d->ldaux; g.scale = d->scale; g.colsum = d->colsum; g.W32 = d->W32; g.W16 = d->W16;
     g.lr = d->lr; g.gout = d->gout; g.lossacc = d->lossacc;
     int bv = 0;
-    int rc = tune_gemm(dev, g, iterations, &bv, best_us);
+    int rc = tune_gemm(dev, g, iterations, &bv, best_us, true);
     if (rc == AH_OK && best_variant) *best_variant = bv;
     return rc;
 }

@@ -219,7 +219,9 @@ int ah_gemm(ah_device *dev, const ah_gemm_desc *d);
  * describes (iterations launches each, after one warm-up, on the device stream with hipEvents; two passes,
  * each variant timed by the lower of its two means), returns
  * the fastest and its mean time, and caches the choice on the device: later launches of the same
- * (ta, tb, M, N, K) with variant 0 use it. d is launched as given, so its outputs must be scratch
+ * (ta, tb, M, N, K) with variant 0 use it. Where variant 0 by itself runs a kernel that is no variant (few
+ * tiles, sizes that no tile divides, few outputs) and that kernel is the fastest, *best_variant is 0 and
+ * nothing is cached (for few tiles: past K = 256). d is launched as given, so its outputs must be scratch
  * (the epilogue runs 2 * (iterations + 1) times per variant). Variants without k-groups differ only in
  * tiling and scheduling and accumulate each output over k in the same order (bit-identical results);
  * the k-group variants 10, 11, 15, 25, 28, 31 and 35-38 add two k-halves, which rounds differently in f32 (relative

@@ -859,3 +859,35 @@ def test_gemm16_short_ragged_k(dev, M, N, K):
     got = C.view(np.float16).astype(np.float64)
     acc = (K + 16) * 2.0**-24 * (np.abs(A) @ np.abs(B).T)
     assert np.all(np.abs(got - (A @ B.T) / 3) <= acc / 3 + 2.0**-11 * np.abs(got) * 1.01 + 2.0**-23)
+
+
+@pytest.mark.parametrize("shape", [(0, 0, 32, 4096, 4096), (0, 0, 999, 1000, 2056), (0, 1, 72, 2048, 1024), (8, 64, 4096)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_gemm16_tune_keeps_the_faster_automatic_choice(dev, shape, tmp_path):
+    """Where the split or the dot kernel is the fastest, tuning finds it (variant 0), drops an older choice of the shape, and
+    later calls run it: the same bits as before."""
+    ta, tb, M, N, K = shape if len(shape) == 5 else (0, 0) + shape
+    path = tmp_path / "tune.txt"
+    dev.gemm_tune_cache(str(path), True)
+    head = path.read_text().splitlines()[0]
+    A, Bm = q16(RNG.standard_normal((M, K))), q16(RNG.standard_normal((N, K)))
+    Bs = store_operand(Bm, tb)
+    dA, dB, dW = dev.buffer(A.astype(np.float16), L.AH_F16), dev.buffer(Bs.astype(np.float16), L.AH_F16), dev.buffer(M * N)
+    kw = dict(dtype=L.AH_F16, epi=L.EPI_SGD, ta=ta, tb=tb, M=M, N=N, K=K, A=dA, B=dB, lda=K, ldb=Bs.shape[1], ldc=N, scale=1.0,
+              W32=dW, lr=-1.0)
+
+    def bits():
+        dW.write(np.zeros(M * N, np.float32))
+        dev.gemm(**kw)
+        return dW.read().view(np.uint32)
+
+    want, key = bits(), f"1/{ta}/{tb}/{M}/{N}/{K}"
+    path.write_text(f"{head}\n{key} 1\n")
+    dev.gemm_tune_cache(str(path), False)
+    best, us = dev.gemm_tune(iterations=3, **kw)
+    assert best == 0 and us > 0
+    np.testing.assert_array_equal(bits(), want)
+    dev.gemm_tune_cache(str(path), True)
+    assert not any(line.startswith(key + " ") for line in path.read_text().splitlines())
+    for b in (dA, dB, dW):
+        b.free()
