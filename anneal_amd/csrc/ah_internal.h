@@ -49,6 +49,8 @@ struct TemplateKernel {
 struct GemmDesc;
 // A contraction launched with the device's tuned f16 variant when the descriptor leaves the choice open.
 hipError_t gemm_dispatch(ah_device *dev, const GemmDesc &g);
+// The f16 variant gemm_dispatch runs for a descriptor that leaves the choice open (0: a kernel that is none).
+int gemm16_open_variant(ah_device *dev, const GemmDesc &g);
 
 }  // namespace ah
 

@@ -23,7 +23,10 @@
 // a value-identity guard that drops any candidate whose output is not bit-identical to the unmodified
 // kernel's on fixed inputs (beam.go:410-451), and a cache keyed by the kernel (here the FNV-64a hash of
 // its template key, epilogue and shape included) holding the winning Opts and the hash of the
-// specialised key (beam.go:100-215).
+// specialised key (beam.go:100-215). The search starts from the key's own kernel: where an open key runs
+// a variant that the seam does not edit from, also from the sequence that leads there. A key that runs the
+// f16 split or dot kernel, which no variant stands for and which adds K in an order of its own, has no
+// candidate with its bits: the search returns the key.
 #include <math.h>
 #include <stdio.h>
 #include <string.h>
@@ -94,6 +97,22 @@ int seam_variant(const GemmDesc &d) {
     return (long)((d.M + 255) / 256) * ((d.N + 255) / 256) >= 224 ? 3 : 1;
 }
 
+// The contraction a gemm key describes, operands aligned and dense (symbolic sizes: 4096).
+GemmDesc key_desc(const std::unordered_map<std::string, std::string> &kv) {
+    GemmDesc d;
+    memset(&d, 0, sizeof d);
+    auto dim = [&](const char *k) { auto it = kv.find(k); return it == kv.end() || it->second == "sym" ? 4096 : atoi(it->second.c_str()); };
+    d.dtype = GEMM_F16;
+    d.M = dim("M"); d.N = dim("N"); d.K = dim("K");
+    d.ta = (int)geti(kv, "ta", 0); d.tb = (int)geti(kv, "tb", 0);
+    auto e = kv.find("epi");
+    const std::string epi = e == kv.end() ? "store" : e->second;
+    d.epi = epi == "bias" ? EPI_BIAS : epi == "bias_relu" ? EPI_BIAS_RELU : epi == "mse" ? EPI_MSE : epi == "mask" ? EPI_MASK
+          : epi == "sgd" || epi == "grad" ? EPI_SGD : EPI_STORE;
+    d.lda = d.ta ? d.M : d.K; d.ldb = d.tb ? d.N : d.K; d.ldc = d.ldaux = d.N;
+    return d;
+}
+
 // Parses a gemm key and its current parameters (variant 0: seam_variant).
 int key_info(const std::string &key, KeyInfo *ki) {
     if (key.compare(0, 5, "tmpl:") != 0) return set_error(AH_ERR_UNSUPPORTED, "opts: not a template key");
@@ -103,13 +122,7 @@ int key_info(const std::string &key, KeyInfo *ki) {
     ki->knobs.f16 = dt != ki->kv.end() && dt->second == "f16";
     if (ki->knobs.f16) {
         int v = (int)geti(ki->kv, "variant", 0);
-        if (v == 0) {
-            GemmDesc d;
-            memset(&d, 0, sizeof d);
-            auto dim = [&](const char *k) { auto it = ki->kv.find(k); return it == ki->kv.end() || it->second == "sym" ? 4096 : atoi(it->second.c_str()); };
-            d.M = dim("M"); d.N = dim("N");
-            v = seam_variant(d);
-        }
+        if (v == 0) v = seam_variant(key_desc(ki->kv));
         if (!gemm16_variant_params(v, &ki->knobs.p)) return set_error(AH_ERR_INVALID, "opts: variant %d", v);
         G16Params &p = ki->knobs.p;
         if (p.fetch <= 3) p.fetch = 0;   // compiler-scheduled class
@@ -267,6 +280,29 @@ std::vector<ah_opt> action_space(const KeyInfo &ki, const Knobs &from) {
     return out;
 }
 
+// The shortest sequence from ki's parameters to f16 variant v through instantiated kernels; empty if there is none.
+std::vector<ah_opt> opts_to_variant(const KeyInfo &ki, int v, Knobs *end) {
+    struct Node {
+        Knobs k;
+        std::vector<ah_opt> opts;
+    };
+    std::vector<Node> q{{ki.knobs, {}}};
+    for (size_t i = 0; i < q.size(); i++) {
+        if (f16_variant_of(q[i].k.p) == v) {
+            *end = q[i].k;
+            return q[i].opts;
+        }
+        if ((int)q[i].opts.size() >= kMaxBeamOpts / 2) continue;
+        for (const ah_opt &o : action_space(ki, q[i].k)) {
+            Node n = q[i];
+            apply_opt(n.k, o);
+            n.opts.push_back(o);
+            if (std::none_of(q.begin(), q.end(), [&](const Node &m) { return m.k == n.k; })) q.push_back(n);
+        }
+    }
+    return {};
+}
+
 int apply_opts_key(const std::string &key, const ah_opt *opts, int n, std::string *out) {
     KeyInfo ki;
     if (int rc = key_info(key, &ki)) return rc;
@@ -418,6 +454,12 @@ int ah_beam_search(ah_device *d, const ah_exec_item *item, int32_t width, int32_
     if (int rc = run_single(d, *item, key.c_str(), in, &ref)) return rc;
     Cand best{{}, ki.knobs, base_us};
     std::vector<Cand> cur{best};
+    if (ki.name == "gemm" && ki.knobs.f16 && geti(ki.kv, "variant", 0) == 0) {
+        Cand own{{}, ki.knobs, base_us};   // the kernel the open key runs, as a sequence
+        const int v = gemm16_open_variant(d, key_desc(ki.kv));
+        if (v) own.opts = opts_to_variant(ki, v, &own.knobs);
+        if (!own.opts.empty()) cur.push_back(own);
+    }
     // a winning sequence holds at most kMaxBeamOpts opts: what ah_beam_result reports and what the cache
     // file's loader accepts
     depth = std::min(depth, kMaxBeamOpts);
@@ -425,6 +467,7 @@ int ah_beam_search(ah_device *d, const ah_exec_item *item, int32_t width, int32_
         std::vector<Cand> next;
         for (const Cand &c : cur) {
             for (const ah_opt &a : action_space(ki, c.knobs)) {
+                if ((int)c.opts.size() >= kMaxBeamOpts) break;
                 Cand n = c;
                 apply_opt(n.knobs, a);
                 n.opts.push_back(a);

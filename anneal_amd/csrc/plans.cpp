@@ -185,6 +185,12 @@ static hipError_t gemm_run(ah_device *dev, GemmDesc g, hipStream_t s) {
 
 hipError_t ah::gemm_dispatch(ah_device *dev, const GemmDesc &g) { return gemm_run(dev, g, dev->stream); }
 
+int ah::gemm16_open_variant(ah_device *dev, const GemmDesc &g) {
+    auto it = dev->gemm_variant.find(tune_key(g));
+    if (it != dev->gemm_variant.end()) return it->second;
+    return gemm16_beside_variants(g) || g.K % 64 ? 0 : gemm16_default_variant(g);
+}
+
 // Times every f16 variant of g (as given: its epilogue runs on whatever outputs g names) and caches
 // the fastest for g's shape. Two passes over the variants, each variant's time the lower of its two
 // means of `iters` launches, so one disturbed measurement does not decide the choice.

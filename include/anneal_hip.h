@@ -276,7 +276,9 @@ typedef struct {
 /* BeamSearch (beam.go:271-408) over item (a "tmpl:" item, buffers as for ah_benchmark): beam width and
  * depth, each candidate timed by ah_benchmark (warmup, iters; min), kept only if its output is
  * bit-identical to the unmodified kernel's on fixed inputs (beam.go:410-451). The winner is cached per
- * process keyed by the FNV-64a hash of the item's key; a cached kernel is re-timed, not searched. */
+ * process keyed by the FNV-64a hash of the item's key; a cached kernel is re-timed, not searched. A key
+ * that runs the f16 split or dot kernel (see ah_gemm_tune) has no candidate with its bits: the winner is
+ * the key itself. */
 int ah_beam_search(ah_device *dev, const ah_exec_item *item, int32_t width, int32_t depth, int32_t warmup,
                    int32_t iters, ah_beam_result *out);
 /* BeamApplyToItems' cache hit (beam.go:470-541): the cached specialised key for key, or key itself; the

@@ -54,3 +54,22 @@ def test_beam_search_value_guard_cache_and_apply(dev, case, tmp_path):
     beam_cache(path, False)
     assert beam_apply(key) == best
     beam_reset()
+
+
+def test_beam_starts_from_the_kernel_the_key_runs(dev):
+    """An open f16 key of 128 tiles and a long K runs a variant of two k-groups, which the seam reaches by a sequence of Opts;
+    only two-k-group kernels have its bits. The search edits that sequence: several candidates pass the guard, and whatever
+    wins has the key's bits."""
+    shape = (1024, 2048, 1024)
+    key = "tmpl:gemm;dtype=f16;epi=store;ta=0;tb=0;M=1024;N=2048;K=1024"
+    beam_reset()
+    item = gemm_item(key, L.AH_F16, shape)
+    r = beam_search(dev, item, width=2, depth=1, warmup=1, iters=3)
+    assert r.searched >= 3 and r.min_us <= r.base_us + 1e-9 and len(r.opts) <= 8
+    M, N, K = shape
+    rng = np.random.default_rng(5)
+    a, b = rng.standard_normal(M * K).astype(np.float32), rng.standard_normal(N * K).astype(np.float32)
+    ex = Executor(dev)
+    want, got = (ex.run([gemm_item(k, L.AH_F16, shape)], {1: a, 2: b})[10] for k in (key, apply_opts(key, r.opts)))
+    np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+    beam_reset()
