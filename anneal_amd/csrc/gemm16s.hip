@@ -78,19 +78,28 @@ static bool choose(const GemmDesc &d, G16SPlan *best) {
 // Where the line lies. The whole-tile variants keep the outputs whose tiles they fill whole (256x256 where those number at
 // least 224, else 128x128; K a multiple of 64) from 64 128x128 tiles up: 2048 x 1024 x 2048 21.7 / 21.9 / 24.3 us there
 // against 19.9 / 23.2 / 24.0 here (NT / N,MN / MN,MN), 2048 x 2048 x 2048 24.5 / 25.2 / 30.9 against 27.4 / 32.3 / 32.0,
-// 4096 x 4096 x 2048 62 / 68 / 105 against 75 / 88 / 104. (Between 64 and 96 tiles this kernel is
-// the faster one, 1024 x 1024 x 2048 16.0 / 17.3 / 17.7 us against 21.2 / 21.3 / 23.2, but adds K in another order than the
-// variants the BEAM search may substitute for an unedited key, which it takes only bit for bit.)
-// They also keep ragged outputs of both operands along K (NT) whose epilogue reads no matrix: only the edge tiles then store
-// element by element. 3584 x 7040 x 128 22.8 us there against 31.1 here, 6709 x 6656 x 320 58.8 against 71.7, 905 x 5120 x 1088
-// 21.9 against 27.4, over 256 tiles on average 1.13 times faster (0.89 to 1.36, 80 shapes); over 192 tiles up to K = 1280
-// (923 x 3840 x 128 7.2 against 9.0), over 128 with K from 384 (3477 x 768 x 640 12.7 against 14.8); with fewer tiles, or a
-// longer K, K split here gains. A K of less than two stages that 64 does not divide goes to the register-staged kernel's 64x64
-// tiles from 65 to 192 128x128 ones: 256 x 5696 x 32 4.6 us against 5.7, 1044 x 1088 x 56 5.1 against 6.0, 2014 x 1816 x 104 on
-// even (1.12 times faster over 45 shapes; below and above the two are within 3%). In the other layouts or with a mask or SGD epilogue this kernel takes half the time.
+// 4096 x 4096 x 2048 62 / 68 / 105 against 75 / 88 / 104. (Between 64 and 96 tiles this kernel is the faster one, 1024 x 1024 x
+// 2048 16.0 / 17.3 / 17.7 us against 21.2 / 21.3 / 23.2. They stay there so that a BEAM search over a key of 64 tiles and more
+// has candidates: it takes only kernels that add K in the open key's order, and none adds it in this one's.)
+//
+// They also keep ragged outputs whose epilogue reads no matrix, as only the edge tiles then store element by element; with a
+// mask or SGD epilogue they take 1.1 to 2 times as long as this kernel.
+//  - Both operands along K (NT): over 256 tiles on average 1.13 times faster (0.89 to 1.36, 80 shapes: 3584 x 7040 x 128 22.8
+//    us there against 31.1, 6709 x 6656 x 320 58.8 against 71.7, 905 x 5120 x 1088 21.9 against 27.4), over 192 tiles up to
+//    K = 1280 (923 x 3840 x 128 7.2 against 9.0), over 128 with K from 384 (3477 x 768 x 640 12.7 against 14.8). With fewer
+//    tiles or a longer K splitting K gains.
+//  - The other layouts: over 192 tiles up to K = 192, 257 to 400 up to K = 1280, each 1.05 to 1.16 times faster on average
+//    over 48 shapes (3904 x 1280 x 256 N,MN 10.3 against 12.5); beyond, 0.77 to 1.02 times.
 static bool whole_tiles(const GemmDesc &d, long t128) {
-    if (d.K % 64 || d.ta || d.tb || d.epi == EPI_MASK || d.epi == EPI_SGD) return false;
+    if (d.K % 64 || d.epi == EPI_MASK || d.epi == EPI_SGD) return false;
+    if (d.ta || d.tb) return t128 > 192 && (d.K <= 192 || (t128 > 256 && t128 <= 400 && d.K <= 1280));
     return t128 > 256 || (d.K <= 1280 && (t128 > 192 || (t128 > 128 && d.K >= 384)));
+}
+// A K of less than two stages that 64 does not divide goes to the register-staged kernel's 64x64 tiles from 65 to 192 128x128
+// ones (NT, likewise): 256 x 5696 x 32 4.6 us there against 5.7, 1044 x 1088 x 56 5.1 against 6.0, 2014 x 1816 x 104 on even, 1.12
+// times faster over 45 shapes; with fewer or more tiles the two are within 3%.
+static bool register_staged(const GemmDesc &d, long t128) {
+    return !d.ta && !d.tb && d.epi != EPI_MASK && d.epi != EPI_SGD && d.K < 128 && d.K % 64 && t128 > 64 && t128 <= 192;
 }
 
 bool gemm16s_serves(const GemmDesc &d) {
@@ -103,8 +112,7 @@ bool gemm16s_serves(const GemmDesc &d) {
     const bool aligned = d.ldc % 4 == 0 && d.ldaux % 4 == 0 && (al & 15) == 0;
     if (aligned && t128 >= 64 && d.M % tile == 0 && d.N % tile == 0 && d.K % 64 == 0) return false;
     if (aligned && whole_tiles(d, t128)) return false;
-    if (!d.ta && !d.tb && d.epi != EPI_MASK && d.epi != EPI_SGD && d.K < 128 && d.K % 64 && t128 > 64 && t128 <= 192) return false;
-    return true;
+    return !register_staged(d, t128);
 }
 
 bool gemm16s_try_launch(const GemmDesc &d, hipStream_t s, hipError_t *err) {

@@ -848,6 +848,38 @@ def test_gemm16_ragged_nt_takes_whole_tiles(dev, M, N, K, variant):
     np.testing.assert_array_equal(C, gemm16_bits(dev, M, N, K, variant=variant, store=True))
 
 
+@pytest.mark.parametrize("shape", [(0, 1, 2440, 2056, 1152), (1, 1, 2440, 2056, 1152), (0, 1, 2000, 2056, 192), (1, 1, 2000, 2056, 192)],
+                         ids=lambda s: "ta%d_tb%d_%dx%dx%d" % s)
+def test_gemm16_ragged_stores_take_whole_tiles(dev, shape):
+    """The same for a plain store in the other layouts, up to their line in K and tiles."""
+    ta, tb, M, N, K = shape
+    np.testing.assert_array_equal(gemm16_bits(dev, M, N, K, ta, tb, store=True), gemm16_bits(dev, M, N, K, ta, tb, variant=1, store=True))
+
+
+@pytest.mark.parametrize("shape", [(0, 0, 905, 5120, 1088), (0, 0, 6709, 6656, 320), (0, 1, 3904, 1280, 256)],
+                         ids=lambda s: "ta%d_tb%d_%dx%dx%d" % s)
+def test_gemm16_ragged_stores_are_no_slower_than_whole_tiles(dev, shape):
+    """An open ragged store takes no longer than the whole-tile kernel its size had before the split one (1.22 to 1.25 times as
+    long where the split kernel took it)."""
+    ta, tb, M, N, K = shape
+    kw = dict(dtype=L.AH_F16, epi=L.EPI_STORE, ta=ta, tb=tb, M=M, N=N, K=K, A=dev.buffer(M * K, L.AH_F16), B=dev.buffer(N * K, L.AH_F16),
+              lda=K, ldb=N if tb else K, C_out=dev.buffer(M * N, L.AH_F16), ldc=N)
+
+    def us(variant):
+        best = 1e9
+        for _ in range(6):
+            dev.timer_start()
+            for _ in range(30):
+                dev.gemm(variant=variant, **kw)
+            best = min(best, dev.timer_stop() / 30 * 1e3)
+        return best
+
+    whole = us(3 if M * N > 224 * 65536 else 1)
+    assert us(0) < 1.1 * whole
+    for k in ("A", "B", "C_out"):
+        kw[k].free()
+
+
 @pytest.mark.parametrize("M,N,K", [(256, 5696, 32), (1044, 1088, 56), (2100, 1500, 104), (1153, 1024, 8)])
 def test_gemm16_short_ragged_k(dev, M, N, K):
     """A short K that 64 does not divide, 65 to 192 tiles: the register-staged kernel's bits (which a fixed variant runs here, as
