@@ -77,7 +77,7 @@ struct ah_device {
     float *chain_scratch = nullptr;
     // This handle's counters of the chain's strip kernel (chain_sync_max_ints, zero between launches), for ah_chain_step_noalloc.
     int *chain_sync = nullptr;
-    // Split-K workspace of the f32 tiled contractions (counters, then partial tiles), set up by ah_open.
+    // Split-K workspace of the f32 tiled and the f16 split contractions (counters, then partial tiles), set up by ah_open.
     void *splitk_ws = nullptr;
     // Loss workspace of ah_softmax_ce (kSoftmaxWsFloats), after the split-K partial tiles in the same allocation (chain_sync
     // follows it): its kernels run in this handle's stream order.

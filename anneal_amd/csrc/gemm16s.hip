@@ -84,16 +84,18 @@ static bool choose(const GemmDesc &d, G16SPlan *best) {
 //
 // They also keep ragged outputs whose epilogue reads no matrix, as only the edge tiles then store element by element; with a
 // mask or SGD epilogue they take 1.1 to 2 times as long as this kernel.
-//  - Both operands along K (NT): over 256 tiles on average 1.13 times faster (0.89 to 1.36, 80 shapes: 3584 x 7040 x 128 22.8
+//  - Both operands along K (NT): over 272 tiles on average 1.13 times faster (0.92 to 1.36, 75 shapes: 3584 x 7040 x 128 22.8
 //    us there against 31.1, 6709 x 6656 x 320 58.8 against 71.7, 905 x 5120 x 1088 21.9 against 27.4), over 192 tiles up to
 //    K = 1280 (923 x 3840 x 128 7.2 against 9.0), over 128 with K from 384 (3477 x 768 x 640 12.7 against 14.8). With fewer
-//    tiles or a longer K splitting K gains.
+//    tiles or a longer K splitting K gains, and past K = 512 with 257 to 272 tiles, which variant 1 puts one to nearly every
+//    CU with two stages in flight (3769 x 1056 x 896 18.1 against 16.6; 727 x 5512 x 320 11.5 against 15.1).
 //  - The other layouts: over 192 tiles up to K = 192, 257 to 400 up to K = 1280, each 1.05 to 1.16 times faster on average
 //    over 48 shapes (3904 x 1280 x 256 N,MN 10.3 against 12.5); beyond, 0.77 to 1.02 times.
 static bool whole_tiles(const GemmDesc &d, long t128) {
     if (d.K % 64 || d.epi == EPI_MASK || d.epi == EPI_SGD) return false;
     if (d.ta || d.tb) return t128 > 192 && (d.K <= 192 || (t128 > 256 && t128 <= 400 && d.K <= 1280));
-    return t128 > 256 || (d.K <= 1280 && (t128 > 192 || (t128 > 128 && d.K >= 384)));
+    if (t128 > 256) return t128 > 272 || d.K <= 512;
+    return d.K <= 1280 && (t128 > 192 || (t128 > 128 && d.K >= 384));
 }
 // A K of less than two stages that 64 does not divide goes to the register-staged kernel's 64x64 tiles from 65 to 192 128x128
 // ones (NT, likewise): 256 x 5696 x 32 4.6 us there against 5.7, 1044 x 1088 x 56 5.1 against 6.0, 2014 x 1816 x 104 on even, 1.12

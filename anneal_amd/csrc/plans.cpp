@@ -757,8 +757,9 @@ struct Mlp3Trainer : ah_trainer {
                 if (gemm16_variant_params(v, &p) && p.kg == 1 && t[v] < t[one]) one = v;
             }
             // On an output of few tiles (up to 32 of 128x128: a few microseconds) one and two k-groups time alike, and
-            // which one wins is noise; they round differently, so one k-group is kept unless two are clearly faster: the
-            // step's bits then do not depend on the timing.
+            // which one wins is mostly noise; they round differently, so one k-group is kept unless two are more than 8%
+            // faster: the step's bits then seldom depend on the timing. (They still do where two k-groups measure about
+            // that much faster, on larger outputs, and on contractions that share a key, which keep the first stage's.)
             const GemmDesc g = gemm(i, false);
             if ((long)((g.M + 127) / 128) * ((g.N + 127) / 128) <= 32 && t[one] <= 1.08 * t[bv]) bv = one;
             dev->gemm_variant[keys[i]] = bv;

@@ -1,7 +1,8 @@
 """ah_chain_step_noalloc (the config-5 chain with its workspace in the library's per-GPU static array)
 against ah_chain_step (the same kernels with a hipMalloc'd workspace), through the C ABI: two calls in a
 row, the second on a smaller input, so a stale workspace from the first call would show. The chain writes
-every workspace entry before reading it, so the two must agree bit for bit."""
+every workspace entry before reading it, so the two must agree bit for bit. The strip kernel's counters, zero between
+calls, lie with each device handle."""
 import numpy as np
 import pytest
 
