@@ -665,7 +665,7 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
     __shared__ __attribute__((aligned(1024))) floatx4 held[kLds > 0 ? kLds : 1][kStripThreads];
     __shared__ float red[4][kStripWaves][kStripCols];
     __shared__ float pstat[4][kParts][kStripCols];
-    __shared__ __attribute__((aligned(16))) float coef[5][kStripCols];   // dX factors A, B, column max, tie share, loss term
+    __shared__ __attribute__((aligned(16))) float coef[6][kStripCols];   // dX factors A, B, column max, tie share, loss term, dg
     __shared__ int flag;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nstrips = (Cc + kStripCols - 1) / kStripCols;
@@ -687,7 +687,6 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
     const long org = (long)rbeg * Cc + c0;
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void *)(X + org), (short)0, 0x7fffffff, 0x00020000);
     const __amdgpu_buffer_rsrc_t dr = __builtin_amdgcn_make_buffer_rsrc((void *)(dX + org), (short)0, 0x7fffffff, 0x00020000);
-    const float gi = tid < kStripCols && c0 + tid < Cc ? g[c0 + tid] : 0.0f;   // before this part arrives
     const int voff = colok ? (rl * Cc + 4 * q) * 4 : kOut, voff0 = ok0 ? (row0 * Cc + 4 * q) * 4 : kOut;
     const int rstepB = kStripRows * Cc * 4;
     // 1. the rows: register slots first (they are consumed first), then the LDS slots
@@ -750,18 +749,19 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
     __syncthreads();
     // 3. the part's column statistics, and the other parts'
     float own[4];
-    int reads = 0, leader = 1;   // thread 0: this part has said that it reads X; wave 0: this part stores dg
     if (tid < kStripCols) strip_fold(kStripWaves, [&](int k, int w) { return red[k][w][tid]; }, own);
     if (parts > 1) {
         float *const mine = stats + ((long)strip * parts + part) * (4 * kStripCols);
         int *const arrive = sync + 2 * strip;
         if (wave == 0) {
+            const float gi = lane < kStripCols && c0 + lane < Cc ? g[c0 + lane] : 0.0f;   // before this part arrives
             if (lane < kStripCols)
 #pragma unroll
                 for (int k = 0; k < 4; k++)
                     __hip_atomic_store(mine + k * kStripCols + lane, own[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             // performed where the XCDs are coherent, before the arrival; g has been read
             asm volatile("s_waitcnt vmcnt(0)" :: "v"(gi) : "memory");
+            if (lane < kStripCols) coef[4][lane] = gi;
             if (lane == 0) {
                 const int all = (1 << parts) - 1;
                 int got = __hip_atomic_fetch_add(arrive, 1 << part, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) | 1 << part;
@@ -769,40 +769,32 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
                     __builtin_amdgcn_s_sleep(4);
                     got = __hip_atomic_load(arrive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
-                reads = (got & all) != all;
+                const bool reads = (got & all) != all;
                 if (reads) got = __hip_atomic_fetch_add(arrive, kStripReader, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                flag = all & ~got;
+                flag = (all & ~got) | (reads ? kStripReader : 0);
             }
         }
         __syncthreads();
-        const int missing = flag;
-        if (missing == 0) {
-            // one value a thread and pass, every load in flight at once (a thread that took its column's parts one after the
-            // other paid 1.1 us a part: 8192 x 64 in 16 parts: 26.4 us, so 11.3)
-            constexpr int kPer = kParts * 4 * kStripCols / kStripThreads;
-            const float *const all = stats + (long)strip * parts * (4 * kStripCols);
-            float got[kPer];
+        const int missing = __builtin_amdgcn_readfirstlane(flag);   // parts, and kStripReader where this one has said that it reads
+        // one value a thread and pass, every load in flight at once (a thread that took its column's parts one after the
+        // other paid 1.1 us a part: 8192 x 64 in 16 parts: 26.4 us, so 11.3)
+        constexpr int kPer = kParts * 4 * kStripCols / kStripThreads;
+        const float *const all = stats + (long)strip * parts * (4 * kStripCols);
+        float got[kPer];
 #pragma unroll
-            for (int j = 0; j < kPer; j++)
-                got[j] = tid + j * kStripThreads < parts * 4 * kStripCols
-                             ? __hip_atomic_load(all + tid + j * kStripThreads, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0f;
+        for (int j = 0; j < kPer; j++)
+            got[j] = tid + j * kStripThreads < parts * 4 * kStripCols
+                         ? __hip_atomic_load(all + tid + j * kStripThreads, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0f;
 #pragma unroll
-            for (int j = 0; j < kPer; j++) {
-                const int i = tid + j * kStripThreads;
-                pstat[i / kStripCols % 4][i / (4 * kStripCols)][i % kStripCols] = got[j];
-            }
-            __syncthreads();
-        } else {
-            // those that are there; the others from X, slot for slot in the order their own workgroup takes them
+        for (int j = 0; j < kPer; j++) {
+            const int i = tid + j * kStripThreads;
+            pstat[i / kStripCols % 4][i / (4 * kStripCols)][i % kStripCols] = got[j];
+        }
+        __syncthreads();
+        if (missing & (kStripReader - 1)) {
+            // the missing ones from X, slot for slot in the order their own workgroup takes them
             for (int p = 0; p < parts; p++) {
-                if ((missing >> p & 1) == 0) {
-                    if (tid < kStripCols)
-#pragma unroll
-                        for (int k = 0; k < 4; k++)
-                            pstat[k][p][tid] = __hip_atomic_load(stats + (((long)strip * parts + p) * 4 + k) * kStripCols + tid,
-                                                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    continue;
-                }
+                if ((missing >> p & 1) == 0) continue;
                 const int pb = p * part_rows, pr = min(part_rows, R - pb), pf = (pr - 1) / kStripRows, r0 = pf * kStripRows + rl;
                 const bool pok = r0 < pr && colok;
                 const float *const px = X + (long)pb * Cc + col;
@@ -838,19 +830,11 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
         if (tid < kStripCols) strip_fold(parts, [&](int k, int p) { return pstat[k][p][tid]; }, own);
         if (tid == 0) {
             // every thread has its values of X by the fold's last barrier
-            if (reads) __hip_atomic_fetch_add(arrive, -kStripReader, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (missing >= kStripReader) __hip_atomic_fetch_add(arrive, -kStripReader, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (in_place)
                 for (int k = 0; k < kStripReaderSpin && __hip_atomic_load(arrive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= kStripReader; k++)
                     __builtin_amdgcn_s_sleep(4);
-            // the last part to leave (every one has arrived by then) clears the words for the next launch
-            const int gone = __hip_atomic_fetch_add(arrive + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            leader = gone == parts - 1;
-            if (leader) {
-                __hip_atomic_store(arrive, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(arrive + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
         }
-        leader = __shfl(leader, 0, 64);   // to wave 0, whose lanes hold the columns
     }
     // 4. the column's scalars (chain_finalize's rules), the same in every part
     if (tid < kStripCols) {
@@ -864,6 +848,7 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
         const float qm = sqq * rR;
         const float T = sqrtf(qm + eps);
         const float r = 1.0f / T;
+        const float gi = parts > 1 ? coef[4][tid] : live ? g[c] : 0.0f;
         const float gR = gi * sumS;
         const float gT = ((-gR) * r) * r;
         const float gu = gT * (1.0f / (2.0f * T));
@@ -879,9 +864,20 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
         coef[2][tid] = mm;
         coef[3][tid] = gm * (1.0f / t_);
         coef[4][tid] = live ? gi * (r * sumS) : 0.0f;
-        if (leader && live) dg[c] = r * sumS;
+        coef[5][tid] = r * sumS;
+        if (parts == 1 && live) dg[c] = r * sumS;
     }
     __syncthreads();
+    // the last part to leave (every one has arrived by then) stores dg and clears the words for the next launch; the other
+    // waves go on meanwhile
+    if (parts > 1 && wave == 0) {
+        int gone = 0;
+        if (lane == 0) gone = __hip_atomic_fetch_add(sync + 2 * strip + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (__builtin_amdgcn_readfirstlane(gone) == parts - 1) {
+            if (lane < kStripCols && c0 + lane < Cc) dg[c0 + lane] = coef[5][lane];
+            if (lane < 2) __hip_atomic_store(sync + 2 * strip + lane, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
     // 5. dX from the held rows
     {
         const floatx4 a = *(const floatx4 *)&coef[0][4 * q], b = *(const floatx4 *)&coef[1][4 * q],
