@@ -555,9 +555,10 @@ __device__ __forceinline__ float strip_tree_sum(float v) {
 
 // A thread's running statistics of its four columns: the reference mt its exponentials are taken against (finite: -FLT_MAX
 // or above, so that an entry of -inf adds exp2(-inf) = 0), sum e, sum e^2 and the exact running max, from -FLT_MAX. An
-// element more than 2^60 above mt (where e^2 could overflow) first moves the reference to itself. The elements equal to the max are counted afterwards, and only where a lane met its running max again (a bit of
-// `tie`, kept in scalar registers): counting them as they land took 5 of 17 vector operations per element, in a kernel whose
-// vector work shows (8192 x 4096: 67.3 us with the count, 59.1 us without any statistics).
+// element more than 2^60 above mt (where e^2 could overflow) first moves the reference to itself. The elements equal to the
+// max are counted afterwards, and only where a lane met its running max again (a bit of `tie`, kept in scalar registers):
+// counting them as they land took 5 of 17 vector operations per element, in a kernel whose vector work shows (8192 x 4096:
+// 67.3 us with the count, 59.1 us without any statistics).
 struct StripStat {
     float mt[4], se[4], sq[4], mr[4];
     uint64_t tie;
