@@ -304,8 +304,8 @@ int ah_chain_step(ah_device *dev, const float *X, const float *g, int32_t R, int
  * allocate device memory (code under HIP graph capture, tight serving loops). The chain's workspace is a
  * file-scope device array of 2^22 floats (16 MiB per GPU, held until the process ends), so
  * 64 + ceil(R/64)*Cc*4 + Cc*8 + ceil(Cc/16) must not exceed 2^22 (config 5, 8192 x 4096, needs 2.13M);
- * larger shapes fail with AH_ERR_INVALID. Asynchronous: the chain's kernel (three where X does not fit on
- * chip) is enqueued on the device stream and the call returns (ah_sync waits). Every call on one GPU
+ * larger shapes fail with AH_ERR_INVALID. Asynchronous: the chain's kernel (three for shapes that do not
+ * fit on chip in one round of workgroups) is enqueued on the device stream and the call returns (ah_sync waits). Every call on one GPU
  * shares that GPU's workspace, so calls of several device handles that overlap on one GPU race: their
  * outputs are undefined (those of later calls are not, as the kernel's counters are each handle's). */
 int ah_chain_step_noalloc(ah_device *dev, const float *X, const float *g, int32_t R, int32_t Cc, float *dX,
