@@ -656,8 +656,10 @@ __device__ __forceinline__ bool strip_in(int i, int nfull) {
 
 // part_rows: rows per part (a multiple of 64, at most 64 * NS; the last part may have fewer). stats: parts * 128 floats a
 // strip. sync: two words a strip, arrivals and departures, zero before and after. in_place: dX or dg shares memory with X or g.
-template <int NS>
-__global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float *X, int R, int Cc, int parts, int part_rows,
+// Up to 16 slots two workgroups share a CU: 4 waves a SIMD, 128 VGPRs. MULTI: more than one part a strip (a strip of one part
+// that jumps over the exchange's code takes 0.4 us more: 630 x 276 10.3 us for 9.8).
+template <int NS, bool MULTI>
+__global__ __launch_bounds__(kStripThreads, NS <= 16 ? 4 : 2) void chain_strip_kernel(const float *X, int R, int Cc, int parts, int part_rows,
                                                                      const float *g, float *dX, float *dg, float *stats,
                                                                      int *sync, float *lossp, int *counter, float *loss,
                                                                      int spin, int in_place) {
@@ -665,7 +667,7 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
     constexpr int kParts = NS > kStripMaxRegs ? kStripMaxPartsFull : kStripMaxParts;
     __shared__ __attribute__((aligned(1024))) floatx4 held[kLds > 0 ? kLds : 1][kStripThreads];
     __shared__ float red[4][kStripWaves][kStripCols];
-    __shared__ float pstat[4][kParts][kStripCols];
+    __shared__ float pstat[4][MULTI ? kParts : 1][kStripCols];
     __shared__ __attribute__((aligned(16))) float coef[6][kStripCols];   // dX factors A, B, column max, tie share, loss term, dg
     __shared__ int flag;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -674,7 +676,7 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
     // no multiple of 32, meet in one L2
     const int L = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
     if (L >= nstrips * parts) return;
-    const int strip = L / parts, part = L - strip * parts;
+    const int strip = MULTI ? L / parts : L, part = L - strip * parts;
     const int q = tid & 7, rl = tid >> 3, c0 = strip * kStripCols, col = c0 + 4 * q;
     const bool colok = col < Cc;   // Cc % 4 == 0: all four columns or none
     const int rbeg = part * part_rows, rows = min(part_rows, R - rbeg), nfull = (rows - 1) / kStripRows;
@@ -688,6 +690,7 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
     const long org = (long)rbeg * Cc + c0;
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void *)(X + org), (short)0, 0x7fffffff, 0x00020000);
     const __amdgpu_buffer_rsrc_t dr = __builtin_amdgcn_make_buffer_rsrc((void *)(dX + org), (short)0, 0x7fffffff, 0x00020000);
+    const float gi = tid < kStripCols && c0 + tid < Cc ? g[c0 + tid] : 0.0f;   // before this part arrives
     const int voff = colok ? (rl * Cc + 4 * q) * 4 : kOut, voff0 = ok0 ? (row0 * Cc + 4 * q) * 4 : kOut;
     const int rstepB = kStripRows * Cc * 4;
     // 1. the rows: register slots first (they are consumed first), then the LDS slots
@@ -751,18 +754,16 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
     // 3. the part's column statistics, and the other parts'
     float own[4];
     if (tid < kStripCols) strip_fold(kStripWaves, [&](int k, int w) { return red[k][w][tid]; }, own);
-    if (parts > 1) {
+    if constexpr (MULTI) {
         float *const mine = stats + ((long)strip * parts + part) * (4 * kStripCols);
         int *const arrive = sync + 2 * strip;
         if (wave == 0) {
-            const float gi = lane < kStripCols && c0 + lane < Cc ? g[c0 + lane] : 0.0f;   // before this part arrives
             if (lane < kStripCols)
 #pragma unroll
                 for (int k = 0; k < 4; k++)
                     __hip_atomic_store(mine + k * kStripCols + lane, own[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             // performed where the XCDs are coherent, before the arrival; g has been read
             asm volatile("s_waitcnt vmcnt(0)" :: "v"(gi) : "memory");
-            if (lane < kStripCols) coef[4][lane] = gi;
             if (lane == 0) {
                 const int all = (1 << parts) - 1;
                 int got = __hip_atomic_fetch_add(arrive, 1 << part, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) | 1 << part;
@@ -849,7 +850,6 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
         const float qm = sqq * rR;
         const float T = sqrtf(qm + eps);
         const float r = 1.0f / T;
-        const float gi = parts > 1 ? coef[4][tid] : live ? g[c] : 0.0f;
         const float gR = gi * sumS;
         const float gT = ((-gR) * r) * r;
         const float gu = gT * (1.0f / (2.0f * T));
@@ -866,12 +866,12 @@ __global__ __launch_bounds__(kStripThreads) void chain_strip_kernel(const float 
         coef[3][tid] = gm * (1.0f / t_);
         coef[4][tid] = live ? gi * (r * sumS) : 0.0f;
         coef[5][tid] = r * sumS;
-        if (parts == 1 && live) dg[c] = r * sumS;
+        if (!MULTI && live) dg[c] = r * sumS;
     }
     __syncthreads();
-    // the last part to leave (every one has arrived by then) stores dg and clears the words for the next launch; the other
-    // waves go on meanwhile
-    if (parts > 1 && wave == 0) {
+    // the last part to leave (every one has arrived by then) stores dg and clears the words for the next launch: one wave's
+    // work, not wave 0's, which takes the loss's ticket behind its stores
+    if (MULTI && wave == kStripWaves - 1) {
         int gone = 0;
         if (lane == 0) gone = __hip_atomic_fetch_add(sync + 2 * strip + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (__builtin_amdgcn_readfirstlane(gone) == parts - 1) {
@@ -979,12 +979,18 @@ bool chain_resident_fits(int R, int Cc) {
     return !rounds || (Cc % kStripCols == 0 && (long)R * Cc * 4 > 250000000L);
 }
 
+template <int NS, bool MULTI>
+static void launch_strip_t(const float *X, const float *g, int R, int Cc, const StripPlan &p, float *stats, int *sync,
+                           float *lossp, int *counter, float *dX, float *dg, float *loss, int spin, int in_place, hipStream_t s) {
+    const int wgs = (Cc + kStripCols - 1) / kStripCols * p.parts;
+    hipLaunchKernelGGL((chain_strip_kernel<NS, MULTI>), dim3((wgs + 7) / 8 * 8), dim3(kStripThreads), 0, s, X, R, Cc, p.parts, p.rows, g,
+                       dX, dg, stats, sync, lossp, counter, loss, spin, in_place);
+}
 template <int NS>
 static void launch_strip(const float *X, const float *g, int R, int Cc, const StripPlan &p, float *stats, int *sync, float *lossp,
                          int *counter, float *dX, float *dg, float *loss, int spin, int in_place, hipStream_t s) {
-    const int wgs = (Cc + kStripCols - 1) / kStripCols * p.parts;
-    hipLaunchKernelGGL(chain_strip_kernel<NS>, dim3((wgs + 7) / 8 * 8), dim3(kStripThreads), 0, s, X, R, Cc, p.parts, p.rows, g,
-                       dX, dg, stats, sync, lossp, counter, loss, spin, in_place);
+    if (p.parts > 1) launch_strip_t<NS, true>(X, g, R, Cc, p, stats, sync, lossp, counter, dX, dg, loss, spin, in_place, s);
+    else launch_strip_t<NS, false>(X, g, R, Cc, p, stats, sync, lossp, counter, dX, dg, loss, spin, in_place, s);
 }
 
 hipError_t chain_resident(const float *X, const float *g, int R, int Cc, float *arrays, int *sync, int *counter, float *dX,
